@@ -341,6 +341,40 @@ def test_moe_more_types(gu, dn):
         assert O.rel_l2(yn, want) <= 5e-3, (gu, dn)
 
 
+@pytest.mark.parametrize("gu,dn", [(Q4K, Q6K), (ggml.GGML_TYPE_Q5_K, Q80), (Q80, Q4K), (Q6K, ggml.GGML_TYPE_Q5_K)])
+@pytest.mark.parametrize("counts", [(300, 1, 0, 83), (256, 129, 112, 15), (33, 48, 65, 192), (64, 160, 100, 20)])
+def test_moe_prefill_tiles(gu, dn, counts):
+    """Prefill-sized batches: every tile height of the expert-grouped kernels
+    (1 .. 16 blocks of 16 slots, experts split into two tiles, an idle expert,
+    last blocks with 1 to 16 live rows), a gate/up K of one and a down K of
+    three super-blocks; with top-2 and top-3 a random routing.  The bound is
+    the other MoE tests': fp16 operands and hidden rows."""
+    from qblocks import rand_qblocks
+    e_n, h, i, t = len(counts), 256, 768, sum(counts)
+
+    def mk(qt, rows, k, seed):
+        return QTensor.from_bytes(rand_qblocks(qt, rows, k, seed), qt, rows, k)
+    gates = [mk(gu, i, h, 400 + e) for e in range(e_n)]
+    ups = [mk(gu, i, h, 500 + e) for e in range(e_n)]
+    downs = [mk(dn, h, i, 600 + e) for e in range(e_n)]
+    rng = np.random.default_rng(gu + dn + counts[0])
+    # the hidden rows are fp16 (below 65504): with these blocks they reach
+    # 1.4e5 at x ~ 0.05 (Q6_K gate/up) and grow with the square of x
+    x = (rng.standard_normal((t, h)) * 0.01).astype(np.float32)
+    want_e = rng.permutation(np.repeat(np.arange(e_n), counts))
+    lg = np.where(np.arange(e_n)[None, :] == want_e[:, None], 3.0, -1.0).astype(np.float32)
+    cases = [(x, lg, 1)] + [(x[:1024 // k], rng.standard_normal((min(t, 1024 // k), e_n)).astype(np.float32), k)
+                            for k in (2, 3)]
+    for xs, l, topk in cases:
+        y, idx, w = moe_grouped_ffn(gates, ups, downs, xs, l, topk)
+        want, widx, ww = moe_oracle(gates, ups, downs, xs, l, topk)
+        assert np.array_equal(idx.cpu().numpy(), widx)
+        assert np.allclose(w.cpu().numpy(), ww, rtol=1e-5, atol=1e-6)
+        yn = y.cpu().numpy()
+        assert np.all(np.isfinite(yn))
+        assert O.rel_l2(yn, want) <= 5e-3, (topk, O.rel_l2(yn, want))
+
+
 @pytest.mark.parametrize("dn", [Q4K, Q6K])
 @pytest.mark.parametrize("topk", [1, 2, 3])
 def test_moe_combine_paths(dn, topk):

@@ -34,6 +34,19 @@ constexpr int MOE_MAX_EXPERTS = 64;
 constexpr int MOE_MAX_TOPK = 8;
 constexpr int MOE_MAX_SLOTS = 1024;  // tokens * topk
 
+// Whether the experts run on moe_wreg.hip, which decodes each weight once per
+// up to 256 slots but cannot fill the chip with a small down product (its
+// workgroups take 128 of the h columns of one expert).  MI355X, Q4_K gate/up
+// and Q6_K down, mean slots per expert in brackets: 8 experts of 4096 x 14336
+// 304 us against 307 at [12], 297 / 412 [16], 314 / 656 [32], 477 / 2168
+// [125]; 32 of 2048 x 4096, top-4, 190 / 201 [8], 194 / 318 [16], 212 / 510
+// [31]; 4 of 2048 x 8192 (64 down workgroups) 107 / 76 [16], 111 / 107 [25].
+bool moe_wreg_shape(int64_t slots, int64_t n_exp, int64_t h) {
+    const int64_t wgs = n_exp * (h / 128);
+    const int64_t per = wgs >= 128 ? 16 : (wgs >= 64 ? 32 : 64);
+    return slots >= per * n_exp;
+}
+
 struct ExpertPtrs {
     const uint8_t* p[MOE_MAX_EXPERTS];
 };
@@ -258,9 +271,9 @@ __global__ void __launch_bounds__(256) moe_down_kernel(ExpertPtrs wd, const floa
 
 // ---- Q4_K experts: skinny tiles (skinny_core.hpp) --------------------------
 //
-// prep: block 0 routes every token once and writes the routing (ridx, rw)
-// and the slots of each expert in slot order (elist[eoff[e] .. eoff[e+1]));
-// the other blocks round x to fp16 (xh) -- the MFMA path rounds its
+// prep: the first blocks route every token once and write the routing (ridx,
+// rw) and the slots of each expert in slot order (elist[eoff[e] ..
+// eoff[e+1]); above 64 slots moe_lists_kernel does); the others round x to fp16 (xh) -- the MFMA path rounds its
 // activations to fp16 anyway, and fp16 halves the activation traffic of the
 // expert kernels.
 constexpr int PREP_THREADS = 1024;
@@ -269,9 +282,9 @@ __global__ void __launch_bounds__(PREP_THREADS) moe_prep_kernel(
         const float* __restrict__ x, const float* __restrict__ logits, int t_n, int e_n, int topk, int64_t nx,
         _Float16* __restrict__ xh, int32_t* __restrict__ ridx, float* __restrict__ rw, int32_t* __restrict__ eoff,
         int32_t* __restrict__ elist, float* __restrict__ yzero, int32_t* __restrict__ out_idx,
-        float* __restrict__ out_w) {
-    if (blockIdx.x > 0) {
-        const int64_t i8 = (static_cast<int64_t>(blockIdx.x - 1) * PREP_THREADS + threadIdx.x) * 8;
+        float* __restrict__ out_w, int rblocks) {
+    if (static_cast<int>(blockIdx.x) >= rblocks) {
+        const int64_t i8 = (static_cast<int64_t>(static_cast<int>(blockIdx.x) - rblocks) * PREP_THREADS + threadIdx.x) * 8;
         if (i8 < nx) {  // nx = t_n * h, a multiple of 256
             const float4 a = *reinterpret_cast<const float4*>(x + i8);
             const float4 b = *reinterpret_cast<const float4*>(x + i8 + 4);
@@ -285,61 +298,84 @@ __global__ void __launch_bounds__(PREP_THREADS) moe_prep_kernel(
         }
         return;
     }
-    __shared__ int sexp[MOE_MAX_SLOTS];
-    __shared__ int scnt[MOE_MAX_EXPERTS + 1];
+    __shared__ int sexp[64];
     const int nslots = t_n * topk;
     // one wave per token
     // with yzero no combine launch follows, and the routing result goes to
     // out_idx / out_w here
     int32_t* const cidx = yzero ? out_idx : nullptr;
     float* const cw = yzero ? out_w : nullptr;
-    for (int t = static_cast<int>(threadIdx.x >> 6); t < t_n; t += PREP_THREADS / 64)
+    for (int t = static_cast<int>(blockIdx.x) * (PREP_THREADS / 64) + static_cast<int>(threadIdx.x >> 6); t < t_n;
+         t += PREP_THREADS / 64 * rblocks)
         route_token_wave(logits + static_cast<int64_t>(t) * e_n, e_n, topk, ridx + t * topk, rw + t * topk,
-                         sexp + t * topk, cidx ? cidx + t * topk : nullptr, cw ? cw + t * topk : nullptr);
+                         rblocks == 1 ? sexp + t * topk : nullptr, cidx ? cidx + t * topk : nullptr,
+                         cw ? cw + t * topk : nullptr);
+    if (rblocks > 1) return;  // the lists follow in moe_lists_kernel
     __syncthreads();
-    if (nslots <= 64) {
-        // one wave: expert e's slots are the lanes whose expert is e; a
-        // ballot per expert gives its count, the running total its offset,
-        // and the lanes below a slot with the same expert its position
-        // (slot order, as the loops below)
-        if (threadIdx.x < 64) {
-            const int q = static_cast<int>(threadIdx.x);
-            const int eq = q < nslots ? sexp[q] : -1;
-            const uint64_t below = (uint64_t(1) << q) - 1u;
-            int total = 0, my_off = 0, my_pos = -1;
-            for (int e = 0; e < e_n; e++) {
-                const uint64_t m = __ballot(eq == e);
-                if (q == e) my_off = total;
-                if (eq == e) my_pos = total + __popcll(m & below);
-                total += __popcll(m);
-            }
-            if (q < e_n) eoff[q] = my_off;
-            if (q == 0) eoff[e_n] = total;
-            if (my_pos >= 0) elist[my_pos] = q;
+    // one wave: expert e's slots are the lanes whose expert is e; a ballot
+    // per expert gives its count, the running total its offset, and the
+    // lanes below a slot with the same expert its position (slot order)
+    if (threadIdx.x < 64) {
+        const int q = static_cast<int>(threadIdx.x);
+        const int eq = q < nslots ? sexp[q] : -1;
+        const uint64_t below = (uint64_t(1) << q) - 1u;
+        int total = 0, my_off = 0, my_pos = -1;
+        for (int e = 0; e < e_n; e++) {
+            const uint64_t m = __ballot(eq == e);
+            if (q == e) my_off = total;
+            if (eq == e) my_pos = total + __popcll(m & below);
+            total += __popcll(m);
         }
-        return;
+        if (q < e_n) eoff[q] = my_off;
+        if (q == 0) eoff[e_n] = total;
+        if (my_pos >= 0) elist[my_pos] = q;
     }
-    // counts per expert, then exclusive offsets (slots with no expert -- NaN
-    // logits -- are in no list)
-    if (threadIdx.x < e_n) {
+}
+
+// The slot lists of more than 64 slots (at most 1024: one thread per slot),
+// in slot order: per wave a ballot per expert gives the counts of its 64
+// slots and each slot's position among them; the counts of the waves before,
+// and of the experts before, make it the slot's place.  Slots with no expert
+// (NaN logits) are in no list.  (A loop over all slots per expert and per
+// slot, with the routing in the same single workgroup, ran 94 us at 500
+// tokens, 8 experts, top-2; the two launches 7.2 + 2.6.)
+__global__ void __launch_bounds__(MOE_MAX_SLOTS) moe_lists_kernel(const int32_t* __restrict__ ridx, int nslots, int e_n,
+                                                                  int32_t* __restrict__ eoff,
+                                                                  int32_t* __restrict__ elist) {
+    constexpr int WAVES = MOE_MAX_SLOTS / 64;
+    __shared__ int cnt[WAVES][MOE_MAX_EXPERTS];
+    __shared__ int off[MOE_MAX_EXPERTS + 1];
+    const int q = static_cast<int>(threadIdx.x), lane = q & 63, wave = q >> 6;
+    const int eq = q < nslots ? ridx[q] : -1;
+    const uint64_t below = (uint64_t(1) << lane) - 1u;
+    int pos = 0, mine = 0;
+    for (int e = 0; e < e_n; e++) {
+        const uint64_t m = __ballot(eq == e);
+        if (eq == e) pos = __popcll(m & below);
+        if (lane == e) mine = __popcll(m);
+    }
+    cnt[wave][lane] = mine;  // lanes past the experts: 0
+    __syncthreads();
+    if (wave == 0) {  // lane e: expert e's counts to the waves' first places
         int c = 0;
-        for (int q = 0; q < nslots; q++) c += sexp[q] == static_cast<int>(threadIdx.x);
-        scnt[threadIdx.x + 1] = c;
+#pragma unroll
+        for (int v = 0; v < WAVES; v++) {
+            const int x = cnt[v][lane];
+            cnt[v][lane] = c;
+            c += x;
+        }
+        int s = c;  // inclusive sum over the experts
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int a = __shfl_up(s, o, 64);
+            if (lane >= o) s += a;
+        }
+        off[lane] = s - c;
+        if (lane < e_n) eoff[lane] = s - c;
+        if (lane == 63) eoff[e_n] = s;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        scnt[0] = 0;
-        for (int e = 0; e < e_n; e++) scnt[e + 1] += scnt[e];
-        for (int e = 0; e <= e_n; e++) eoff[e] = scnt[e];
-    }
-    __syncthreads();
-    for (int q = threadIdx.x; q < nslots; q += PREP_THREADS) {
-        const int e = sexp[q];
-        if (e < 0 || e >= e_n) continue;
-        int pos = 0;
-        for (int r = 0; r < q; r++) pos += sexp[r] == e;
-        elist[scnt[e] + pos] = q;
-    }
+    if (eq >= 0 && eq < e_n) elist[off[eq] + cnt[wave][eq] + pos] = q;
 }
 
 // gate/up: grid (ceil(i / 64), E).  A workgroup streams 64 rows of the
@@ -564,15 +600,23 @@ extern "C" int vb_moe_grouped_ffn_types(const void* const* wg, const void* const
     int32_t* eoff = reinterpret_cast<int32_t*>(wsb + ws.eoff);
     int32_t* elist = reinterpret_cast<int32_t*>(wsb + ws.elist);
     // 1. routing, per-expert slot lists, fp16 activations
-    const dim3 prep(static_cast<uint32_t>(1 + (nx / 8 + PREP_THREADS - 1) / PREP_THREADS));
+    // one routing workgroup and its lists up to 64 slots; above, a wave per
+    // token over as many workgroups as that takes and the lists in a launch of
+    // their own
+    const int rblocks = slots <= 64 ? 1 : static_cast<int>((n_tokens + PREP_THREADS / 64 - 1) / (PREP_THREADS / 64)) + 1;
+    const dim3 prep(static_cast<uint32_t>(rblocks + (nx / 8 + PREP_THREADS - 1) / PREP_THREADS));
     // top-k <= 2 on the quantized experts: the down kernels add each slot's
     // weighted output into y (zeroed here), so no combine launch follows
     const bool fused_combine = !f32 && topk <= 2;
     float* yacc = fused_combine ? y : nullptr;
     moe_prep_kernel<<<prep, dim3(PREP_THREADS), 0, st>>>(x, router_logits, n_tokens, n_exp, topk, nx, xh, ridx, rw,
-                                                         eoff, elist, yacc, out_idx, out_w);
+                                                         eoff, elist, yacc, out_idx, out_w, rblocks);
     int rc = check_launch("vb_moe_grouped_ffn");
     if (rc != OK) return rc;
+    if (rblocks > 1) {
+        moe_lists_kernel<<<dim3(1), dim3(MOE_MAX_SLOTS), 0, st>>>(ridx, static_cast<int>(slots), n_exp, eoff, elist);
+        if ((rc = check_launch("vb_moe_grouped_ffn")) != OK) return rc;
+    }
     // 2, 3. experts
     if (!f32) {
         const int64_t rb_gu = row_bytes(gate_up_type, h), rb_d = row_bytes(down_type, i);
@@ -585,7 +629,15 @@ extern "C" int vb_moe_grouped_ffn_types(const void* const* wg, const void* const
         // serves four 16-row column groups); the other types on the
         // expert-grouped K-split kernel (gemm_kq.hip), gate/up with the same
         // SwiGLU epilogue
-        if (gate_up_type == TYPE_Q4_K) {
+        const bool wreg = moe_wreg_type(gate_up_type) && moe_wreg_type(down_type) &&
+                          moe_wreg_shape(slots, n_exp, h);
+        if (wreg) {
+            // the packed rows (at most slots + 15 n_exp <= 2 slots of them)
+            // take obuf's place until the down product writes it
+            rc = moe_wreg(gate_up_type, down_type, wg, wu, wd, n_exp, xh, static_cast<int>(slots), topk, h, i, eoff,
+                          elist, obuf, hb16, obuf, rw, yacc, st);
+            if (rc != OK) return rc;
+        } else if (gate_up_type == TYPE_Q4_K) {
             const dim3 gu(static_cast<uint32_t>((i + skinny::ROWS - 1) / skinny::ROWS), n_exp);
             moe_gate_up_q4k<MOE_WAVES><<<gu, dim3(64 * MOE_WAVES), skinny::lds_bytes<MOE_WAVES>(), st>>>(
                 pg, pu, xh, eoff, elist, static_cast<int>(slots), topk, static_cast<int>(h), static_cast<int>(i),
@@ -596,7 +648,8 @@ extern "C" int vb_moe_grouped_ffn_types(const void* const* wg, const void* const
                                 static_cast<int>(slots), i, h, hb16, nullptr, nullptr, nullptr, st)) != OK) {
             return rc;
         }
-        if (down_type == TYPE_Q4_K) {
+        if (wreg) {
+        } else if (down_type == TYPE_Q4_K) {
             const dim3 dn(static_cast<uint32_t>((h + skinny::ROWS - 1) / skinny::ROWS), n_exp);
             moe_down_q4k<MOE_WAVES><<<dn, dim3(64 * MOE_WAVES), skinny::lds_bytes<MOE_WAVES>(), st>>>(
                 pd, hb16, eoff, elist, static_cast<int>(slots), static_cast<int>(h), static_cast<int>(i),

@@ -184,6 +184,16 @@ constexpr int MOE_KQ_MAX_EXPERTS = 64;
 int moe_kq(int32_t type, bool gate_up, const void* const* w0, const void* const* w1, int n_exp, const void* X,
            int64_t xbytes, int topk, const int32_t* eoff, const int32_t* elist, int nslots, int64_t N, int64_t K,
            _Float16* hout, float* fout, const float* rw, float* yacc, hipStream_t st);
+// The same products for prefill-sized batches (moe_wreg.hip): each expert's
+// weights read and decoded once per 256 slots, for the types moe_wreg_type
+// takes on both sides, h and i multiples of 256.  xh: the tokens in fp16.
+// xf / hf: scratch of (nslots + 15 n_exp) x h (x i) fp16 values (packed
+// activations and hidden rows); with yacc null, obuf (nslots x h fp32, may
+// overlap xf) takes the expert outputs.
+bool moe_wreg_type(int32_t t);
+int moe_wreg(int32_t gu_type, int32_t dn_type, const void* const* wg, const void* const* wu, const void* const* wd,
+             int n_exp, const _Float16* xh, int nslots, int topk, int64_t h, int64_t i, const int32_t* eoff,
+             const int32_t* elist, void* xf, void* hf, float* obuf, const float* rw, float* yacc, hipStream_t st);
 int gemm_dispatch(const void* w, const void* X, int32_t x_dtype, float* Y, int64_t M, int64_t N, int64_t K,
                   int32_t type, int32_t variant, void* ws, size_t ws_bytes, hipStream_t st);
 
