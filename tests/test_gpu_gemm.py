@@ -836,3 +836,54 @@ def test_q5k_xreg(m, n, k):
         assert np.array_equal(gemm(qt, xt).cpu().numpy().view(np.uint32), y.view(np.uint32))
 
 
+
+
+@pytest.mark.parametrize("qtype", [Q4K, ggml.GGML_TYPE_Q5_K, Q6K, Q80])
+@pytest.mark.parametrize("m,n,k", [(2, 300, 256), (16, 128, 2560), (17, 1, 768), (47, 257, 2304), (64, 300, 1024),
+                                   (65, 129, 512), (81, 300, 2048), (97, 300, 256), (113, 140, 2304),
+                                   (129, 300, 1280), (145, 33, 512), (161, 300, 2304), (193, 96, 256),
+                                   (256, 300, 3328)])
+def test_wreg(knob, qtype, m, n, k):
+    """The register-decoding kernel (gemm_wreg.hip) at every tile height, row
+    tiles, K splits of unequal length (13, 9 and 10 super-blocks), K groups
+    with nothing to do (one super-block) and ragged N, both X types."""
+    knob("VB_GEMM_WREG_MIN_M", "2")
+    lib = _lib.load()
+    if qtype == ggml.GGML_TYPE_Q5_K:
+        qt, x = make_other(qtype, n, k, m * 17 + n), make(m, 1, k, m)[1]
+    else:
+        qt, x = make(m, n, k, m * 17 + n + qtype, qtype=qtype)
+    for dtype in (torch.float16, torch.float32):
+        xt = torch.from_numpy(x).to("cuda", dtype)
+        assert lib.vb_gemm_scratch(m, n, k, qtype, 1 if dtype == torch.float16 else 0, 0) >= m * k * 2
+        y = gemm(qt, xt).cpu().numpy()
+        assert np.all(np.isfinite(y))
+        assert O.rel_l2(y, ref_gemm(qt, xt.float().cpu().numpy())) <= TOL, dtype
+
+
+@pytest.mark.parametrize("qtype,m,n,k,dtype", [(Q4K, 100, 1024, 14336, torch.float16),
+                                               (Q6K, 33, 300, 8192, torch.float16),
+                                               (Q80, 8, 300, 12288, torch.float32),
+                                               (Q6K, 300, 8200, 512, torch.float32),
+                                               (Q4K, 600, 1000, 4096, torch.float32)])
+def test_scratch_routes(qtype, m, n, k, dtype):
+    """Routes that vb_gemm_scratch opens: the register-decoding kernel and
+    fp32 X on the packed-X kernel.  Without a workspace, and with one that is
+    a byte short, the call still runs, and all agree."""
+    lib = _lib.load()
+    qt, x = make(m, n, k, m + n, qtype=qtype)
+    xt = torch.from_numpy(x).to("cuda", dtype)
+    xdt = 1 if dtype == torch.float16 else 0
+    need = lib.vb_gemm_scratch(m, n, k, qtype, xdt, 0)
+    assert need > lib.vb_gemm_workspace(m, n, k, qtype, xdt, 0)
+    want = ref_gemm(qt, xt.float().cpu().numpy())
+    y = gemm(qt, xt).cpu().numpy()
+    assert O.rel_l2(y, want) <= TOL
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    s = torch.cuda.current_stream().cuda_stream
+    for nb in (0, need - 1):
+        out = torch.empty((m, n), dtype=torch.float32, device="cuda")
+        assert lib.vb_gemm_ws(qt.ptr(), xt.data_ptr(), xdt, out.data_ptr(), m, n, k, qtype, 0, ws.data_ptr(), nb,
+                              s) == 0
+        # the same fp16 operands in another order of fp32 sums
+        assert O.rel_l2(out.cpu().numpy(), y) <= 1e-5

@@ -20,9 +20,6 @@
 namespace vb {
 namespace {
 
-constexpr int X_F32 = 0;
-constexpr int X_F16 = 1;
-
 // ---- tiled: M > 16 ------------------------------------------------------------
 //
 // Workgroup tile: TB_M = 64 WM rows of X x BN = 16 * NF weight rows (output
@@ -748,6 +745,25 @@ int gemm_other(const void* w, const void* X, int32_t x_dtype, float* Y, int64_t 
     return rc;
 }
 
+// The packed-X kernel beyond the shapes whose workspace vb_gemm_workspace
+// states, with the splits of gemm_xr_ksplit_even: fp32 X (the tiled kernel
+// converts it once per column tile), and fp16 X at N < 8192 for the types
+// whose other kernels decode slowly.  MI355X, us old / packed-X: fp32 X, Q6_K
+// 4096 x 14336 at M = 777 250 / 163, 14110 x 3072 at 359 125 / 61, Q4_K 14336
+// x 4096 at 512 94 / 64, 1773 x 13056 at 279 144 / 46, 4187 x 4864 at 828 69 /
+// 75, 1024 x 1024 at 300 16 / 22; fp16 X, Q4_0 5461 x 12288 at 533 229 / 131,
+// 5487 x 1536 at 972 53 / 35, 684 x 1536 at 414 16 / 26, Q5_K 7056 x 6400 at
+// 992 122 / 98, 2499 x 1792 at 941 33 / 33 (Q4_K, Q6_K and Q8_0 there keep
+// the tiled kernel: Q8_0 7943 x 8448 at 845 169 / 201).
+static bool xr_even_shape(int32_t type, int32_t x_dtype, int64_t M, int64_t N, int64_t K) {
+    if (!gemm_xr_type(type) || M <= 256 || M > INT32_MAX || K % 256 != 0) return false;
+    const bool b32 = gemm_b32_type(type);
+    if (!b32 && type != TYPE_Q4_K && type != TYPE_Q5_K && !knobs().gemm_xr_kq) return false;
+    if (x_dtype == X_F32) return N * K >= 4000000 && !(type == TYPE_Q4_K && N < 8192 && M > 768);
+    return N < 8192 && gemm_xr_ksplit(M, N, K) == 1 &&
+           ((b32 && N * K >= 8000000) || (type == TYPE_Q5_K && N * K >= 16000000));
+}
+
 int gemm_dispatch(const void* w, const void* X, int32_t x_dtype, float* Y, int64_t M, int64_t N, int64_t K,
                   int32_t type, int32_t variant, void* ws, size_t ws_bytes, hipStream_t st) {
     if (type != TYPE_Q4_K && type != TYPE_Q6_K && type != TYPE_Q8_0 && type != TYPE_Q5_K && !gemm_b32_type(type) &&
@@ -798,6 +814,18 @@ int gemm_dispatch(const void* w, const void* X, int32_t x_dtype, float* Y, int64
         if (type != TYPE_Q4_K && !general && K > 4096 && gemv_split_rpw(type, N, K) > 0)
             return gemv_split(type, w, X, Y, nullptr, N, K, st, true);
     }
+    // with the workspace of vb_gemm_scratch: the register-decoding kernel and
+    // the packed-X kernel past its fixed shapes
+    if (variant == 0 && ws != nullptr && reinterpret_cast<uintptr_t>(ws) % 16 == 0 && N <= INT32_MAX &&
+        M * K * 4 < (int64_t(1) << 32) && ((N * rb + 3) & ~int64_t(3)) < (int64_t(1) << 32)) {
+        const int64_t have = static_cast<int64_t>(ws_bytes);
+        if (gemm_wreg_shape(type, x_dtype, M, N, K) && have >= gemm_wreg_workspace(M, N, K))
+            return gemm_wreg(w, X, x_dtype, Y, M, N, K, type, ws, st);
+        if (xr_even_shape(type, x_dtype, M, N, K)) {
+            const int ks = gemm_xr_ksplit_even(M, N, K);
+            if (have >= gemm_xr_workspace(M, N, K, ks)) return gemm_xr(w, X, x_dtype, Y, M, N, K, type, ws, ks, st);
+        }
+    }
     if (gemm_b32_type(type)) {
         // Q4_0 / Q4_1 / Q5_0 / Q5_1: their decoder in the K-split kernel at
         // small M (variant 4) and in the packed-X kernel for M > 256 with a
@@ -816,10 +844,10 @@ int gemm_dispatch(const void* w, const void* X, int32_t x_dtype, float* Y, int64
                           "of %lld bytes", static_cast<long long>(xr_need));
                 return E_INVAL;
             }
-            return gemm_xr(w, X, Y, M, N, K, type, ws, st);
+            return gemm_xr(w, X, x_dtype, Y, M, N, K, type, ws, gemm_xr_ksplit(M, N, K), st);
         }
         if (variant == 0 && xr_ok && M > 256 && (N >= 8192 || gemm_xr_ksplit(M, N, K) > 1))
-            return gemm_xr(w, X, Y, M, N, K, type, ws, st);
+            return gemm_xr(w, X, x_dtype, Y, M, N, K, type, ws, gemm_xr_ksplit(M, N, K), st);
     }
     bool tiled = false;
     if (gemm_b32_type(type)) {
@@ -952,7 +980,7 @@ int gemm_dispatch(const void* w, const void* X, int32_t x_dtype, float* Y, int64
                          (N >= 8192 || gemm_xr_ksplit(M, N, K) > 1) && ws != nullptr &&
                          static_cast<int64_t>(ws_bytes) >= gemm_xr_workspace(M, N, K) &&
                          reinterpret_cast<uintptr_t>(ws) % 16 == 0;
-    if (xr_auto) return gemm_xr(w, X, Y, M, N, K, type, ws, st);
+    if (xr_auto) return gemm_xr(w, X, x_dtype, Y, M, N, K, type, ws, gemm_xr_ksplit(M, N, K), st);
     if (variant == 5) {
         if (M < 256) {
             set_error("vb_gemm: variant 5 (X in registers) takes m >= 256, got %lld", static_cast<long long>(M));
@@ -964,7 +992,7 @@ int gemm_dispatch(const void* w, const void* X, int32_t x_dtype, float* Y, int64
                       static_cast<long long>(need), ws_bytes);
             return E_INVAL;
         }
-        return gemm_xr(w, X, Y, M, N, K, type, ws, st);
+        return gemm_xr(w, X, x_dtype, Y, M, N, K, type, ws, gemm_xr_ksplit(M, N, K), st);
     }
     if (type == TYPE_Q4_K && (variant == 3 || (variant == 0 && x_dtype == X_F16 && split_range))) {
         return gemm_q4k_split(w, X, Y, M, N, K, st);
@@ -1050,6 +1078,18 @@ extern "C" int64_t vb_gemm_workspace(int64_t m, int64_t n, int64_t k, int32_t gg
         return zs > 1 ? static_cast<int64_t>(zs) * m * n * 4 : 0;
     }
     return 0;
+}
+
+extern "C" int64_t vb_gemm_scratch(int64_t m, int64_t n, int64_t k, int32_t ggml_type, int32_t x_dtype,
+                                   int32_t variant) {
+    const int64_t need = vb_gemm_workspace(m, n, k, ggml_type, x_dtype, variant);
+    if (variant != 0 || k <= 0 || k % 256 != 0 || m <= 0 || n <= 0) return need;
+    if (vb::gemm_wreg_shape(ggml_type, x_dtype, m, n, k)) return vb::gemm_wreg_workspace(m, n, k);
+    if (vb::xr_even_shape(ggml_type, x_dtype, m, n, k)) {
+        const int64_t xr = vb::gemm_xr_workspace(m, n, k, vb::gemm_xr_ksplit_even(m, n, k));
+        return xr > need ? xr : need;
+    }
+    return need;
 }
 
 extern "C" int vb_gemm_ws(const void* w, const void* x, int32_t x_dtype, float* y, int64_t m, int64_t n, int64_t k,

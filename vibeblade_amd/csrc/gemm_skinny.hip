@@ -22,7 +22,7 @@ __global__ void __launch_bounds__(64 * NW) gemm_q4k_skinny_kernel(
         const uint8_t* __restrict__ w, const uint8_t* __restrict__ X, float* __restrict__ Y, int M, int N, int K,
         int rb, int rows, int nsb, uint32_t wbytes, uint32_t xbytes) {
     extern __shared__ skinny::u32x4 sk_lds[];
-    constexpr uint32_t ES = XT == skinny::X_F16 ? 2u : 4u;
+    constexpr uint32_t ES = XT == X_F16 ? 2u : 4u;
     const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
     skinny::TileArgs<1, MT> ta;
     ta.w[0] = skinny::make_rsrc(w, wbytes);
@@ -63,7 +63,7 @@ __global__ void __launch_bounds__(64 * NW) gemm_q4k_skinny_kernel(
 int gemm_q4k_skinny(const void* w, const void* X, int32_t x_dtype, float* Y, int64_t M, int64_t N, int64_t K,
                     hipStream_t st) {
     const int64_t nsb = K / 256, rb = nsb * 144;
-    const int64_t xbytes = M * K * (x_dtype == skinny::X_F16 ? 2 : 4);
+    const int64_t xbytes = M * K * (x_dtype == X_F16 ? 2 : 4);
     if (N > INT32_MAX || K > INT32_MAX || N * rb >= (int64_t(1) << 32) || xbytes >= (int64_t(1) << 31)) {
         set_error("vb_gemm: shape too large for the skinny kernel (N=%lld K=%lld)", static_cast<long long>(N),
                   static_cast<long long>(K));
@@ -81,30 +81,30 @@ int gemm_q4k_skinny(const void* w, const void* X, int32_t x_dtype, float* Y, int
     const uint32_t wbytes = static_cast<uint32_t>(N * rb), xby = static_cast<uint32_t>(xbytes);
     if (M > 32) {
         // four activation tiles (fp16 X): 4-wave workgroups, one per CU
-        if (x_dtype != skinny::X_F16 || M > 64) {
+        if (x_dtype != X_F16 || M > 64) {
             set_error("vb_gemm: the skinny kernel takes M <= 32 (M <= 64 with fp16 X), got %lld",
                       static_cast<long long>(M));
             return E_INVAL;
         }
         constexpr int NW4 = 4;
-        gemm_q4k_skinny_kernel<skinny::X_F16, 4, NW4><<<grid, dim3(64 * NW4), skinny::lds_bytes_mt<NW4, 4, 1>(), st>>>(
+        gemm_q4k_skinny_kernel<X_F16, 4, NW4><<<grid, dim3(64 * NW4), skinny::lds_bytes_mt<NW4, 4, 1>(), st>>>(
             wb, xb, Y, m, n, k, rbi, rowsi, nsbi, wbytes, xby);
     } else if (M > 16) {
         // two activation tiles: 4-wave workgroups (the register file of a
         // SIMD to one wave), one per CU
         constexpr int NW2 = 4;
         const size_t lds2 = skinny::lds_bytes<NW2>();
-        if (x_dtype == skinny::X_F16)
-            gemm_q4k_skinny_kernel<skinny::X_F16, 2, NW2><<<grid, dim3(64 * NW2), lds2, st>>>(
+        if (x_dtype == X_F16)
+            gemm_q4k_skinny_kernel<X_F16, 2, NW2><<<grid, dim3(64 * NW2), lds2, st>>>(
                 wb, xb, Y, m, n, k, rbi, rowsi, nsbi, wbytes, xby);
         else
-            gemm_q4k_skinny_kernel<skinny::X_F32, 2, NW2><<<grid, dim3(64 * NW2), lds2, st>>>(
+            gemm_q4k_skinny_kernel<X_F32, 2, NW2><<<grid, dim3(64 * NW2), lds2, st>>>(
                 wb, xb, Y, m, n, k, rbi, rowsi, nsbi, wbytes, xby);
-    } else if (x_dtype == skinny::X_F16) {
-        gemm_q4k_skinny_kernel<skinny::X_F16, 1, skinny::WAVES><<<grid, block, lds, st>>>(wb, xb, Y, m, n, k, rbi, rowsi,
+    } else if (x_dtype == X_F16) {
+        gemm_q4k_skinny_kernel<X_F16, 1, skinny::WAVES><<<grid, block, lds, st>>>(wb, xb, Y, m, n, k, rbi, rowsi,
                                                                                          nsbi, wbytes, xby);
     } else {
-        gemm_q4k_skinny_kernel<skinny::X_F32, 1, skinny::WAVES><<<grid, block, lds, st>>>(wb, xb, Y, m, n, k, rbi, rowsi,
+        gemm_q4k_skinny_kernel<X_F32, 1, skinny::WAVES><<<grid, block, lds, st>>>(wb, xb, Y, m, n, k, rbi, rowsi,
                                                                                          nsbi, wbytes, xby);
     }
     return check_launch("vb_gemm");

@@ -72,7 +72,7 @@ __device__ __forceinline__ int xr_tile_row0(int t, int M) {
     return r < M - XR_TM ? r : M - XR_TM;
 }
 
-// Pack X (M x K fp16, row-major) into fragment order.  Entry [ks][w][a]
+// Pack X (M x K fp16, or fp32 rounded to fp16, row-major) into fragment order.  Entry [ks][w][a]
 // [lane] of step s of M-tile t (16 bytes) is X[t0 + 64 w + 16 a + lane % 16,
 // 64 s + 32 ks + 8 (lane / 16) .. + 8).  Workgroup (kb, blk, t) moves the
 // 16 x 256 block of rows t0 + 16 blk .. + 16 and elements 256 kb .. + 256:
@@ -80,6 +80,7 @@ __device__ __forceinline__ int xr_tile_row0(int t, int M) {
 // transpose through LDS (rows padded by 16 bytes: the 16 rows a fragment
 // read gathers fall in distinct banks), and 1 KB contiguous stores (one
 // fragment per 64 threads).
+template <int XT>
 __global__ void __launch_bounds__(256) xr_pack_kernel(const uint8_t* __restrict__ X, uint4* __restrict__ Xf,
                                                       int M, int K) {
     __shared__ uint4 tl[16 * 33];
@@ -90,8 +91,7 @@ __global__ void __launch_bounds__(256) xr_pack_kernel(const uint8_t* __restrict_
 #pragma unroll
     for (int q = 0; q < 2; q++) {
         const int idx = q * 256 + tid, row = idx >> 5, piece = idx & 31;
-        tl[row * 33 + piece] =
-            *reinterpret_cast<const uint4*>(X + (static_cast<int64_t>(r0 + row) * K + 256 * kb + 8 * piece) * 2);
+        tl[row * 33 + piece] = x8_f16<XT>(X, static_cast<int64_t>(r0 + row) * K + 256 * kb + 8 * piece);
     }
     __syncthreads();
     uint4* dst = Xf + static_cast<int64_t>(t) * nsteps * (XR_STEP_BYTES / 16);
@@ -544,15 +544,37 @@ int gemm_xr_ksplit(int64_t M, int64_t N, int64_t K) {
     return static_cast<int>(ks < 1 ? 1 : (ks > 8 ? 8 : ks));
 }
 
+// K splits when the output tiles fill the CUs unevenly (4096 x 14336 at M =
+// 777: 37 x 4 tiles on 256 CUs): the count that finishes first, from whole
+// rounds of workgroups, 17 ns per element of K each, and the sum of the
+// partial products.
+int gemm_xr_ksplit_even(int64_t M, int64_t N, int64_t K) {
+    const int64_t tiles = (N + 16 * XR_NF - 1) / (16 * XR_NF) * ((M + XR_TM - 1) / XR_TM), cus = num_cus();
+    int best = 1;
+    double tbest = 0;
+    for (int64_t ks = 1; ks <= 8 && (ks == 1 || K / 256 / ks >= 4); ks++) {
+        const double rounds = static_cast<double>((tiles * ks + cus - 1) / cus);
+        const double t = rounds / ks * 17e-9 * K + (ks > 1 ? 3e-6 + ks * M * N * 8 / 4e12 : 0);
+        if (ks == 1 || t < tbest) {
+            best = static_cast<int>(ks);
+            tbest = t;
+        }
+    }
+    return best;
+}
+
 int gemm_ksum(const float* P, float* Y, int64_t total, int ks, hipStream_t st) {
     xr_ksum_kernel<<<dim3(static_cast<uint32_t>((total / 4 + 255) / 256 + 1)), dim3(256), 0, st>>>(P, Y, total, ks);
     return check_launch("vb_gemm");
 }
 
-int64_t gemm_xr_workspace(int64_t M, int64_t N, int64_t K) {
+int64_t gemm_xr_workspace(int64_t M, int64_t N, int64_t K, int ks) {
     const int64_t xf = (M + XR_TM - 1) / XR_TM * XR_TM * K * 2;
-    const int ks = gemm_xr_ksplit(M, N, K);
     return xf + (ks > 1 ? static_cast<int64_t>(ks) * M * N * 4 : 0);
+}
+
+int64_t gemm_xr_workspace(int64_t M, int64_t N, int64_t K) {
+    return gemm_xr_workspace(M, N, K, gemm_xr_ksplit(M, N, K));
 }
 
 bool gemm_xr_type(int32_t type) {
@@ -565,16 +587,18 @@ bool gemm_xr_type(int32_t type) {
 // dwords, M * K * 2 < 2^32), K % 256 == 0, M >= 256 and the workspace
 // (gemm_xr_workspace bytes, 16-byte aligned): the packed X, then, with K
 // splits, one fp32 M x N partial product per split.
-int gemm_xr(const void* w, const void* X, float* Y, int64_t M, int64_t N, int64_t K, int32_t type, void* ws,
-            hipStream_t st) {
+int gemm_xr(const void* w, const void* X, int32_t x_dtype, float* Y, int64_t M, int64_t N, int64_t K, int32_t type,
+            void* ws, int ks, hipStream_t st) {
     constexpr int NF = XR_NF;
     const int64_t rb = row_bytes(type, K);
     // whole dwords: a Q6_K window's last dword may hold the tensor's last two bytes
     const uint32_t wbytes = static_cast<uint32_t>((N * rb + 3) & ~int64_t(3));
     const uint32_t mtiles = static_cast<uint32_t>((M + XR_TM - 1) / XR_TM);
-    const int ks = gemm_xr_ksplit(M, N, K);
-    xr_pack_kernel<<<dim3(static_cast<uint32_t>(K / 256), XR_TM / 16, mtiles), dim3(256), 0, st>>>(
-        static_cast<const uint8_t*>(X), static_cast<uint4*>(ws), static_cast<int>(M), static_cast<int>(K));
+    const dim3 pg(static_cast<uint32_t>(K / 256), XR_TM / 16, mtiles);
+    const uint8_t* x8 = static_cast<const uint8_t*>(X);
+    uint4* xp = static_cast<uint4*>(ws);
+    if (x_dtype == X_F16) xr_pack_kernel<X_F16><<<pg, dim3(256), 0, st>>>(x8, xp, static_cast<int>(M), static_cast<int>(K));
+    else xr_pack_kernel<X_F32><<<pg, dim3(256), 0, st>>>(x8, xp, static_cast<int>(M), static_cast<int>(K));
     float* out = Y;
     if (ks > 1) out = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + mtiles * XR_TM * K * 2);
     const dim3 grid(static_cast<uint32_t>((N + 16 * NF - 1) / (16 * NF)), mtiles, static_cast<uint32_t>(ks));

@@ -23,6 +23,10 @@
 
 namespace vb {
 
+// x_dtype of the batched products
+constexpr int X_F32 = 0;
+constexpr int X_F16 = 1;
+
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
@@ -72,6 +76,16 @@ __device__ __forceinline__ void f32x8_to_frag_nat(const float4& a, const float4&
     o[1] = pk(a.z, a.w);
     o[2] = pk(b.x, b.y);
     o[3] = pk(b.z, b.w);
+}
+
+// Elements at .. at + 7 of X as fp16 (fp32 rounded).
+template <int XT>
+__device__ __forceinline__ uint4 x8_f16(const void* X, int64_t at) {
+    if constexpr (XT == X_F16) return *reinterpret_cast<const uint4*>(static_cast<const _Float16*>(X) + at);
+    const float4* p = reinterpret_cast<const float4*>(static_cast<const float*>(X) + at);
+    uint32_t o[4];
+    f32x8_to_frag_nat(p[0], p[1], o);
+    return make_uint4(o[0], o[1], o[2], o[3]);
 }
 
 // Per-row scale pair of Q4_K sub-blocks 2c and 2c+1 as fp16 half2 splats:

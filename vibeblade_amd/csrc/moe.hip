@@ -413,7 +413,7 @@ __global__ void __launch_bounds__(64 * NW, NW <= 4 ? 2 : 1) moe_gate_up_q4k(
         ta.xoff[0] = j < nrow ? (static_cast<uint32_t>(slots[m0 + j] / topk) * static_cast<uint32_t>(h) + 64u * g) * 2u
                            : skinny::X_NONE;
         float4_t s[2];
-        skinny::tile<skinny::X_F16, 2, 2, NW, 1, true>(ta, reinterpret_cast<uint8_t*>(moe_lds), s);
+        skinny::tile<X_F16, 2, 2, NW, 1, true>(ta, reinterpret_cast<uint8_t*>(moe_lds), s);
         if (threadIdx.x < 256) {
             const int q = threadIdx.x >> 6, l = threadIdx.x & 63;
             const int r = 16 * q + (l & 15), n = ta.row0 + r;
@@ -458,7 +458,7 @@ __global__ void __launch_bounds__(64 * NW, NW <= 4 ? 2 : 1) moe_down_q4k(
         ta.xoff[0] = j < nrow ? (static_cast<uint32_t>(slots[m0 + j]) * static_cast<uint32_t>(i_dim) + 64u * g) * 2u
                            : skinny::X_NONE;
         float4_t s[1];
-        skinny::tile<skinny::X_F16, 1, 2, NW, 1, true>(ta, reinterpret_cast<uint8_t*>(moe_lds), s);
+        skinny::tile<X_F16, 1, 2, NW, 1, true>(ta, reinterpret_cast<uint8_t*>(moe_lds), s);
         if (threadIdx.x < 256) {
             const int q = threadIdx.x >> 6, l = threadIdx.x & 63;
             const int r = 16 * q + (l & 15), n = ta.row0 + r;

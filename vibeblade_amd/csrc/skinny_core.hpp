@@ -52,8 +52,6 @@ constexpr int lds_bytes_mt() {
     return NW * STAGE > MT * NMAT * NW * 4096 ? NW * STAGE : MT * NMAT * NW * 4096;
 }
 constexpr int LDS_BYTES = lds_bytes<WAVES>();
-constexpr int X_F32 = 0;
-constexpr int X_F16 = 1;
 constexpr uint32_t X_NONE = 0x80000000u;   // lane offset of an absent activation row (reads zeros)
 
 // buffer-load helpers shared with the GEMV (vb_common.hpp)

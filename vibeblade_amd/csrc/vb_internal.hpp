@@ -18,6 +18,7 @@ namespace vb {
 //   VB_GEMM_SPLIT_MIN_M=m                     smallest M (up to 768) on the role-split GEMM (0: never)
 //   VB_GEMM_ZSPLIT=z                          with VB_GEMM_TILE: K splits between workgroups (Q6_K / Q8_0,
 //                                             fp16 X, M >= 384, N < 8192)
+//   VB_GEMM_WREG_MIN_M=m                      smallest M on the register-decoding GEMM (above 256: never)
 //   VB_GEMV_DMA=0                             short- and split-row Q4_K GEMV (fp32 x): register ring
 //                                             instead of LDS DMA
 //   VB_GEMV_SPLIT="sl,d"                      split-row Q4_K GEMV: slices per row (2, 4, 8), rows in flight (1-4)
@@ -38,6 +39,7 @@ struct Knobs {
     int gemm_split_min_m = -1;  // smallest M on the role-split kernel (-1: default)
     int gemm_zsplit = 0;        // with VB_GEMM_TILE: K splits between workgroups (Q6_K / Q8_0)
     bool gemm_xr_kq = true;     // Q6_K / Q8_0 on the packed-X kernel where Q4_K takes it (VB_GEMM_XR_KQ=0: tiled)
+    int gemm_wreg_min_m = -1;   // smallest M on the register-decoding kernel (-1: default)
     int gemv_split_sl = 0, gemv_split_d = 0;  // split-row Q4_K GEMV: slices per row, rows in flight
     bool sparse_fused = true;
     int sparse_npw = 0;
@@ -152,6 +154,8 @@ int gemm_ksum(const float* P, float* Y, int64_t total, int ks, hipStream_t st);
 // K splits of the tiled GEMM between workgroups for this shape (1: none; gemm.hip).
 int tiled_zsplit(int type, int x_dtype, int64_t M, int64_t N, int64_t K);
 int64_t gemm_xr_workspace(int64_t M, int64_t N, int64_t K);
+int gemm_xr_ksplit_even(int64_t M, int64_t N, int64_t K);
+int64_t gemm_xr_workspace(int64_t M, int64_t N, int64_t K, int ks);
 // n_rows x k of W (a decodable type other than F16) as row-major fp16 at out,
 // each value rounded once (dequant.hip; k % 4 == 0, out 16-byte aligned).
 int dequant_rows_f16(const void* w, _Float16* out, int64_t n_rows, int64_t k, int32_t type, hipStream_t st);
@@ -165,8 +169,8 @@ bool gemm_b32_type(int32_t type);
 bool gemm_b32_high(int32_t type);  // Q5_0 / Q5_1
 int64_t gemm_b32_kq_max_m(int64_t N);
 int64_t gemm_other_workspace(int32_t type, int64_t N, int64_t K);
-int gemm_xr(const void* w, const void* X, float* Y, int64_t M, int64_t N, int64_t K, int32_t type, void* ws,
-            hipStream_t st);
+int gemm_xr(const void* w, const void* X, int32_t x_dtype, float* Y, int64_t M, int64_t N, int64_t K, int32_t type,
+            void* ws, int ks, hipStream_t st);
 // Q6_K / Q8_0 GEMM, every M (gemm_kq.hip); pointers, alignment, x_dtype and
 // M, N > 0 already validated.
 int gemm_kq(const void* w, const void* X, int32_t x_dtype, float* Y, int64_t M, int64_t N, int64_t K, int32_t type,
@@ -194,6 +198,14 @@ bool moe_wreg_type(int32_t t);
 int moe_wreg(int32_t gu_type, int32_t dn_type, const void* const* wg, const void* const* wu, const void* const* wd,
              int n_exp, const _Float16* xh, int nslots, int topk, int64_t h, int64_t i, const int32_t* eoff,
              const int32_t* elist, void* xf, void* hf, float* obuf, const float* rw, float* yacc, hipStream_t st);
+// Q4_K / Q5_K / Q6_K / Q8_0 GEMM with the weights decoded once, in registers
+// (gemm_wreg.hip): the shapes variant 0 takes it for, given its workspace
+// (packed X and the partial products of the K splits, 16-byte aligned).  W
+// and X 16-byte aligned and the 32-bit offset bounds validated by the caller.
+bool gemm_wreg_shape(int32_t type, int32_t x_dtype, int64_t M, int64_t N, int64_t K);
+int64_t gemm_wreg_workspace(int64_t M, int64_t N, int64_t K);
+int gemm_wreg(const void* w, const void* X, int32_t x_dtype, float* Y, int64_t M, int64_t N, int64_t K, int32_t type,
+              void* ws, hipStream_t st);
 int gemm_dispatch(const void* w, const void* X, int32_t x_dtype, float* Y, int64_t M, int64_t N, int64_t K,
                   int32_t type, int32_t variant, void* ws, size_t ws_bytes, hipStream_t st);
 

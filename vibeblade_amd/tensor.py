@@ -169,9 +169,9 @@ def gemm(w: QTensor, x: torch.Tensor, out: torch.Tensor | None = None,
     _check_out(out, m * w.rows, w.device, "gemm")
     xdt = X_F16 if x.dtype == torch.float16 else X_F32
     lib = _lib.load()
-    nb = int(lib.vb_gemm_workspace(m, w.rows, w.k, w.qtype, xdt, variant))
+    nb = int(lib.vb_gemm_scratch(m, w.rows, w.k, w.qtype, xdt, variant))
     if nb > 0:
-        # the packed-X kernel's workspace, from torch's caching allocator
+        # packed X and partial products, from torch's caching allocator
         ws = torch.empty(nb, dtype=torch.uint8, device=w.device)
         _lib.call("vb_gemm_ws", w.ptr(), x.data_ptr(), xdt, out.data_ptr(), m, w.rows, w.k, w.qtype,
                   variant, ws.data_ptr(), nb, _stream())
