@@ -189,3 +189,26 @@ def test_predict_and_block_in_a_graph():
         assert torch.equal(g_y, y), rep
         pred.update(0, rng.random(i) < 0.2)  # eager work between replays
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("n", [1, 63, 4096, 4097, 8192, 8193, 16384, 16385, 32768])
+def test_warm_predict_sets(n):
+    """The warm kernel at the edges of its sizes (values per thread) on the
+    values that decide a set: few distinct averages with ties across the
+    k-th, all equal, signed zeros, denormals, infinities, continuous ones;
+    k = 1 to n, thresholds above and below the k-th.  Exact sets."""
+    rng = np.random.default_rng(n)
+    few = rng.choice(np.float32([0, 0, 0, 0.1, 0.19, 0.271, 0.5]), n)
+    zeros = np.where(rng.random(n) < 0.5, np.float32(0.0), np.float32(-0.0)).astype(np.float32)
+    zeros[rng.integers(0, n, max(1, n // 50))] = 1e-42
+    wild = rng.standard_normal(n).astype(np.float32)
+    wild[rng.integers(0, n, max(1, n // 20))] = np.inf
+    wild[rng.integers(0, n, max(1, n // 20))] = -np.inf
+    for probs in (few, zeros, wild, np.full(n, 0.25, np.float32), rng.random(n).astype(np.float32)):
+        for k in sorted({1, max(1, n // 10), max(1, n - 1), n}):
+            for thr in (0.3, 2.0):
+                mask, act, c = _device_predict(probs, k, thr, True)
+                want = probs >= np.float32(thr)
+                want[np.argsort(-probs, kind="stable")[:k]] = True
+                assert np.array_equal(mask, want), (k, thr)
+                assert c == want.sum() and np.array_equal(act, np.flatnonzero(want))

@@ -963,6 +963,181 @@ __global__ void __launch_bounds__(1024) ema_predict_reg_kernel(const float* __re
     if (t == 0) *count = ta;
 }
 
+// ---- warm prediction (n <= 1024 * PER), one workgroup --------------------------
+//
+// top-k(probs) | {probs >= threshold}: the sets ema_predict_kernel selects.
+// Wave w holds elements w * 64 PER .. in registers, lane l of slot j element
+// 64 j + l of them: index order is wave, slot, lane, so a rank is the total
+// of the earlier waves (one exchange of 16 numbers) plus ballots.  Slots past
+// n hold the NaN with the lowest key: never selected before a real element.
+//
+// The k-th key comes from four 8-bit digits.  Averages of few observations
+// take few values and most are zero, so a histogram's atomics pile up on a
+// bin or two: the first digit counts the zeros' digit and the wave's first
+// digit with ballots, and only the others lane by lane; the keys that share
+// the k-th one's first digit go on to a list, and the other three digits read
+// that.  Every wave reads the 256 bins itself (four per lane, one suffix
+// scan), so a digit costs one barrier.
+//
+// Instructions on the one CU bound it: each one spent per element is 0.1 us
+// at n = 14336.  MI355X, k = 1433, a threshold set of 0.08 n, prediction and
+// sparse block of one layer in a graph: 45.6 us with three 11-bit digits over
+// values in LDS (serial bin scans by one wave, ranks over 16 x 16 cells), 29.9
+// now (all four digits over every key: 23.6 us for this launch alone).
+template <int PER>
+__global__ void __launch_bounds__(1024) ema_predict_warm_kernel(const float* __restrict__ probs, int n, int k,
+                                                                float threshold, uint8_t* __restrict__ mask,
+                                                                int32_t* __restrict__ active,
+                                                                int32_t* __restrict__ count) {
+    __shared__ int4 hist[4][64];           // per digit, bins 4 l .. 4 l + 3
+    __shared__ int2 wtot[2][16];           // per wave: sure and tied elements
+    __shared__ uint32_t list[PER * 1024];  // keys with the k-th one's first digit
+    __shared__ int nlist;
+    const int lane = static_cast<int>(threadIdx.x) & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int e0 = wave * PER * 64 + lane;
+    auto below = [](uint64_t b) __attribute__((always_inline)) {
+        return static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(b >> 32),
+                                                          __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(b), 0u)));
+    };
+    float v[PER];
+#pragma unroll
+    for (int j = 0; j < PER; j++) v[j] = e0 + 64 * j < n ? probs[e0 + 64 * j] : __uint_as_float(0xFFFFFFFFu);
+    reinterpret_cast<int*>(hist)[threadIdx.x] = 0;
+    if (threadIdx.x == 0) nlist = 0;
+    int nsure = 0;  // of the wave
+#pragma unroll
+    for (int j = 0; j < PER; j++) nsure += __popcll(__ballot(v[j] >= threshold));
+    if (lane == 0) wtot[0][wave] = make_int2(nsure, 0);
+    __syncthreads();
+    int total = 0;
+#pragma unroll
+    for (int w = 0; w < 16; w++) total += wtot[0][w].x;
+    int ties = 0;
+    uint32_t kth = 0xFFFFFFFFu;
+    const bool need = total < k;  // else the threshold set contains the top k
+    if (need) {
+        // the bin of the k-th key of digit `pass` among the keys counted
+        int rem = k;
+        auto bin_of = [&](int pass) __attribute__((always_inline)) -> uint32_t {
+            const int4 b = hist[pass][lane];
+            const int mine = b.x + b.y + b.z + b.w;
+            int suf = mine;  // over lanes >= this one
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int t = __shfl_down(suf, o, 64);
+                if (lane + o < 64) suf += t;
+            }
+            // keys above each of the lane's bins
+            const int c3 = suf - mine, c2 = c3 + b.w, c1 = c2 + b.z, c0 = c1 + b.y;
+            const int at = c2 >= rem ? 3 : (c1 >= rem ? 2 : (c0 >= rem ? 1 : 0));
+            const int over = at == 3 ? c3 : (at == 2 ? c2 : (at == 1 ? c1 : c0));
+            const int hit = __builtin_ctzll(__ballot(c3 < rem && suf >= rem));
+            rem -= __builtin_amdgcn_readlane(over, hit);
+            return static_cast<uint32_t>(4 * hit + __builtin_amdgcn_readlane(at, hit));
+        };
+        {
+            int* h = reinterpret_cast<int*>(hist[0]);
+            constexpr uint32_t dz = 0x80u;  // zero's digit
+            const uint32_t df = __builtin_amdgcn_readfirstlane(order_key(v[0]) >> 24);
+            int cz = 0, cf = 0;
+#pragma unroll
+            for (int j = 0; j < PER; j++) {
+                const uint32_t d = order_key(v[j]) >> 24;
+                cz += __popcll(__ballot(d == dz));
+                cf += __popcll(__ballot(d == df));
+                if (d != dz && d != df) atomicAdd(h + d, 1);
+            }
+            if (lane == 0) {
+                atomicAdd(h + dz, cz);
+                if (df != dz) atomicAdd(h + df, cf);
+            }
+        }
+        __syncthreads();
+        const uint32_t first = bin_of(0);
+        int c = 0;
+#pragma unroll
+        for (int j = 0; j < PER; j++) c += __popcll(__ballot(order_key(v[j]) >> 24 == first));
+        if (c) {
+            int at = 0;
+            if (lane == 0) at = atomicAdd(&nlist, c);
+            at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+            for (int j = 0; j < PER; j++) {
+                const uint32_t key = order_key(v[j]);
+                const uint64_t m = __ballot(key >> 24 == first);
+                if (m == 0) continue;
+                if (key >> 24 == first) list[at + below(m)] = key;
+                at += __popcll(m);
+            }
+        }
+        __syncthreads();
+        kth = first << 24;
+        const int cnt = nlist;
+#pragma unroll
+        for (int pass = 1; pass < 4; pass++) {
+            const int sh = 24 - 8 * pass;
+            int* h = reinterpret_cast<int*>(hist[pass]);
+            for (int i0 = 64 * wave; i0 < cnt; i0 += 1024) {
+                const int i = i0 + lane;
+                const uint32_t key = i < cnt ? list[i] : 0u;
+                const bool live = i < cnt && (key ^ kth) >> (sh + 8) == 0;
+                const uint64_t m = __ballot(live);
+                if (m == 0) continue;
+                const int d = static_cast<int>((key >> sh) & 255u);
+                const int lead = __builtin_ctzll(m), dl = __builtin_amdgcn_readlane(d, lead);
+                const uint64_t ms = __ballot(live && d == dl);
+                if (lane == lead) atomicAdd(h + dl, __popcll(ms));
+                else if (live && d != dl) atomicAdd(h + d, 1);
+            }
+            __syncthreads();
+            kth |= bin_of(pass) << sh;
+        }
+        ties = rem;  // keys equal to the k-th that belong to the top k, lowest indices first
+        nsure = 0;
+        int ntied = 0;
+#pragma unroll
+        for (int j = 0; j < PER; j++) {
+            const uint32_t key = order_key(v[j]);
+            const bool s = v[j] >= threshold || key > kth;
+            nsure += __popcll(__ballot(s));
+            ntied += __popcll(__ballot(!s && key == kth));
+        }
+        if (lane == 0) wtot[1][wave] = make_int2(nsure, ntied);
+        __syncthreads();
+    }
+    int base = 0, tbase = 0, seen = 0;  // selected and tied elements of the earlier waves
+    total = 0;
+#pragma unroll
+    for (int w = 0; w < 16; w++) {
+        const int2 c = wtot[need ? 1 : 0][w];
+        const int left = ties - seen, took = c.x + (c.y < left ? c.y : (left > 0 ? left : 0));
+        if (w < wave) {
+            base += took;
+            tbase += c.y;
+        }
+        seen += c.y;
+        total += took;
+    }
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const int e = e0 + 64 * j;
+        const uint32_t key = order_key(v[j]);
+        bool s = v[j] >= threshold || (need && key > kth);
+        const bool q = need && !s && key == kth;
+        const uint64_t tb = __ballot(q);
+        if (tb) {
+            s = s || (q && tbase + below(tb) < ties);
+            tbase += __popcll(tb);
+        }
+        const uint64_t sb = __ballot(s);
+        if (s) active[base + below(sb)] = e;
+        if (e < n) mask[e] = s ? 1 : 0;
+        base += __popcll(sb);
+    }
+    if (threadIdx.x == 0) *count = total;
+}
+
 size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
 struct SparseWs {
@@ -1302,9 +1477,18 @@ extern "C" int vb_ema_predict(const float* probs, const float* gate_values, int6
     const int flags = (warm ? PRED_WARM : 0) | (gate_values ? PRED_GATE : 0) | (combined ? PRED_COMBINED : 0);
     const int ni = static_cast<int>(n);
     hipStream_t st = as_stream(stream);
-    // register-resident for n <= 16384 (16 values per thread; 32 would spill
-    // at 1024 threads), the streaming kernel above
-    if (n <= 1024 * 16)
+    // warm and no gate in it: values in registers up to n = 32768; else values
+    // in LDS for n <= 16384, the streaming kernel above
+    if (warm && !combined && n <= 1024 * 32) {
+        auto go = [&](auto per_c) {
+            ema_predict_warm_kernel<decltype(per_c)::value><<<dim3(1), dim3(1024), 0, st>>>(
+                probs, ni, k, threshold, mask_out, active_out, count_out);
+        };
+        if (n <= 1024 * 4) go(std::integral_constant<int, 4>{});
+        else if (n <= 1024 * 8) go(std::integral_constant<int, 8>{});
+        else if (n <= 1024 * 16) go(std::integral_constant<int, 16>{});
+        else go(std::integral_constant<int, 32>{});
+    } else if (n <= 1024 * 16)
         ema_predict_reg_kernel<16><<<dim3(1), dim3(1024), 0, st>>>(probs, gate_values, ni, k, threshold, flags,
                                                                    mask_out, active_out, count_out);
     else
