@@ -887,3 +887,22 @@ def test_scratch_routes(qtype, m, n, k, dtype):
                               s) == 0
         # the same fp16 operands in another order of fp32 sums
         assert O.rel_l2(out.cpu().numpy(), y) <= 1e-5
+
+
+@pytest.mark.parametrize("qtype", [ggml.GGML_TYPE_Q5_K, Q6K, Q80])
+@pytest.mark.parametrize("m,n,k", [(2, 16, 256), (5, 4099, 512), (8, 8200, 768), (16, 333, 4096), (3, 4097, 2304),
+                                   (15, 12300, 1024), (9, 1, 3840)])
+def test_rows(knob, qtype, m, n, k):
+    """The row-streaming kernel (gemm_rows.hip): one to four groups of 16 rows
+    per workgroup with a ragged last one, waves with none to four K steps,
+    rows of every alignment, both X types."""
+    knob("VB_GEMM_ROWS_MIN_N", "1")
+    if qtype == ggml.GGML_TYPE_Q5_K:
+        qt, x = make_other(qtype, n, k, m * 19 + n), make(m, 1, k, m)[1]
+    else:
+        qt, x = make(m, n, k, m * 19 + n + qtype, qtype=qtype)
+    for dtype in (torch.float16, torch.float32):
+        xt = torch.from_numpy(x).to("cuda", dtype)
+        y = gemm(qt, xt).cpu().numpy()
+        assert np.all(np.isfinite(y))
+        assert O.rel_l2(y, ref_gemm(qt, xt.float().cpu().numpy())) <= TOL, dtype

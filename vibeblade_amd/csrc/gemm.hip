@@ -814,6 +814,7 @@ int gemm_dispatch(const void* w, const void* X, int32_t x_dtype, float* Y, int64
         if (type != TYPE_Q4_K && !general && K > 4096 && gemv_split_rpw(type, N, K) > 0)
             return gemv_split(type, w, X, Y, nullptr, N, K, st, true);
     }
+    if (variant == 0 && gemm_rows_shape(type, M, N, K)) return gemm_rows(w, X, x_dtype, Y, M, N, K, type, st);
     // with the workspace of vb_gemm_scratch: the register-decoding kernel and
     // the packed-X kernel past its fixed shapes
     if (variant == 0 && ws != nullptr && reinterpret_cast<uintptr_t>(ws) % 16 == 0 && N <= INT32_MAX &&

@@ -83,6 +83,7 @@ Knobs read_knobs() {
         const int v = std::atoi(e);
         if (v >= 1 && v <= 8) k.gemm_zsplit = v;
     }
+    if (const char* e = std::getenv("VB_GEMM_ROWS_MIN_N")) k.gemm_rows_min_n = std::atoi(e);
     if (const char* e = std::getenv("VB_GEMM_WREG_MIN_M")) k.gemm_wreg_min_m = std::atoi(e);
     if (const char* e = std::getenv("VB_GEMM_XR_KQ")) k.gemm_xr_kq = std::atoi(e) != 0;
     if (const char* e = std::getenv("VB_SPARSE_FUSED")) k.sparse_fused = e[0] != '0';

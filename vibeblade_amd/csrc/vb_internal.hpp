@@ -18,6 +18,7 @@ namespace vb {
 //   VB_GEMM_SPLIT_MIN_M=m                     smallest M (up to 768) on the role-split GEMM (0: never)
 //   VB_GEMM_ZSPLIT=z                          with VB_GEMM_TILE: K splits between workgroups (Q6_K / Q8_0,
 //                                             fp16 X, M >= 384, N < 8192)
+//   VB_GEMM_ROWS_MIN_N=n                      smallest N on the row-streaming GEMM (huge: never)
 //   VB_GEMM_WREG_MIN_M=m                      smallest M on the register-decoding GEMM (above 256: never)
 //   VB_GEMV_DMA=0                             short- and split-row Q4_K GEMV (fp32 x): register ring
 //                                             instead of LDS DMA
@@ -39,6 +40,7 @@ struct Knobs {
     int gemm_split_min_m = -1;  // smallest M on the role-split kernel (-1: default)
     int gemm_zsplit = 0;        // with VB_GEMM_TILE: K splits between workgroups (Q6_K / Q8_0)
     bool gemm_xr_kq = true;     // Q6_K / Q8_0 on the packed-X kernel where Q4_K takes it (VB_GEMM_XR_KQ=0: tiled)
+    int gemm_rows_min_n = -1;   // smallest N on the row-streaming kernel (-1: default)
     int gemm_wreg_min_m = -1;   // smallest M on the register-decoding kernel (-1: default)
     int gemv_split_sl = 0, gemv_split_d = 0;  // split-row Q4_K GEMV: slices per row, rows in flight
     bool sparse_fused = true;
@@ -206,6 +208,12 @@ bool gemm_wreg_shape(int32_t type, int32_t x_dtype, int64_t M, int64_t N, int64_
 int64_t gemm_wreg_workspace(int64_t M, int64_t N, int64_t K);
 int gemm_wreg(const void* w, const void* X, int32_t x_dtype, float* Y, int64_t M, int64_t N, int64_t K, int32_t type,
               void* ws, hipStream_t st);
+// Q5_K / Q6_K / Q8_0 GEMM at 2 <= M <= 16 and K <= 4096 with the weight
+// rows streamed whole through LDS (gemm_rows.hip): the shapes variant 0 takes
+// it for.  W and X 16-byte aligned.
+bool gemm_rows_shape(int32_t type, int64_t M, int64_t N, int64_t K);
+int gemm_rows(const void* w, const void* X, int32_t x_dtype, float* Y, int64_t M, int64_t N, int64_t K, int32_t type,
+              hipStream_t st);
 int gemm_dispatch(const void* w, const void* X, int32_t x_dtype, float* Y, int64_t M, int64_t N, int64_t K,
                   int32_t type, int32_t variant, void* ws, size_t ws_bytes, hipStream_t st);
 
