@@ -20,6 +20,7 @@
 // group's loads in flight bound it.  Q4_K stays on its skinny kernel
 // (gemm_skinny.hip): 83 us against 89 at 128256 x 4096, 11 against 16 at 14336.
 #include "kq_types.hpp"
+#include "tile_index.hpp"
 #include "vb_internal.hpp"
 #include "../../include/vbhip.h"
 
@@ -29,7 +30,6 @@ namespace {
 constexpr int ROWS_WAVES = 8;
 constexpr int ROWS_STEPS = 4;       // 128-element steps per wave, at most
 constexpr int ROWS_MAX_K = 4096;
-constexpr uint32_t ROWS_NONE = 0x80000000u;  // lane offset past every tensor: reads zeros, no traffic
 
 constexpr int rows_block_bytes(int type) {  // of 256 elements
     return type == TYPE_Q5_K ? 176 : (type == TYPE_Q6_K ? 210 : 272);
@@ -69,7 +69,7 @@ __global__ void __launch_bounds__(64 * ROWS_WAVES) gemm_rows_kernel(const uint8_
     const KqConsts kc = kq_consts();
     const int first = static_cast<int>(blockIdx.x), stride = static_cast<int>(gridDim.x);
 
-    // rows 16 grp .. + 15; a group past the last reads nothing
+    // rows 16 grp .. + 15; rows and groups past the last read nothing
     u32x4 st[P];
     const uint32_t pitch = rb + (GAP ? 16u : 0u);
     int at[P];  // the lane's slots in an image; pieces past the rows go to its last one
@@ -79,13 +79,11 @@ __global__ void __launch_bounds__(64 * ROWS_WAVES) gemm_rows_kernel(const uint8_
         at[i] = slot < rb ? static_cast<int>(slot + (GAP ? slot / (rb >> 4) : 0u)) : IMG - 1;
     }
     auto fetch = [&](int grp) __attribute__((always_inline)) {
-        const bool live = grp < ngroups;
-        const uint32_t so = live ? static_cast<uint32_t>(grp) * 16u * rb : 0u;
 #pragma unroll
         for (int i = 0; i < P; i++) {
             const uint32_t slot = static_cast<uint32_t>((wave + ROWS_WAVES * i) * 64 + lane);
-            const uint32_t vo = live && slot < rb ? 16u * slot : ROWS_NONE;
-            st[i] = __builtin_amdgcn_raw_buffer_load_b128(wr, static_cast<int>(vo), static_cast<int>(so), 2);
+            const uint32_t vo = rows_fetch_at(grp, ngroups, slot, rb);
+            st[i] = __builtin_amdgcn_raw_buffer_load_b128(wr, static_cast<int>(vo), 0, 2);
         }
     };
     auto put = [&](u32x4* dst) __attribute__((always_inline)) {
