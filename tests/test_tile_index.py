@@ -42,6 +42,52 @@ int main() {
 }
 """
 
+MOE = r"""
+#include <cstdio>
+#include <initializer_list>
+#include "tile_index.hpp"
+static uint32_t rnd = 1;
+static int next(int n) { rnd = rnd * 1664525u + 1013904223u; return int((rnd >> 8) % uint32_t(n)); }
+// Slot counts of a routing (sum <= nslots): every tile is accepted, the tiles
+// cover the experts' blocks once and number at most moe_wreg_tiles.  Counts
+// each within [0, nslots] but of any sum, as overwritten lists can hold:
+// every accepted tile stays below moe_wreg_blocks.
+int main() {
+    for (int rep = 0; rep < 20000; rep++) {
+        const int n_exp = 1 + next(64), nslots = 1 + next(1024), cap = vb::moe_wreg_blocks(nslots, n_exp);
+        const bool wild = rep & 1;
+        int count[64], left = nslots, first = 0, tiles = 0;
+        for (int e = 0; e < n_exp; e++) {
+            count[e] = wild ? next(nslots + 1) : (e + 1 < n_exp ? next(left + 1) >> next(4) : left);
+            if (!wild) left -= count[e];
+        }
+        for (int mb : {1, 16}) {
+            first = tiles = 0;
+            for (int e = 0; e < n_exp; e++) {
+                const int nb = (count[e] + 15) / 16, nt = (nb + mb - 1) / mb;
+                int blocks = 0, slots = 0;
+                for (int ti = 0; ti < nt; ti++) {
+                    vb::MoeTile t{};
+                    const bool ok = vb::moe_wreg_tile(e, ti, count[e], first, mb, cap, t);
+                    if (ok && (t.blk0 < 0 || t.nblk < 1 || t.nblk > mb || t.blk0 + t.nblk > cap)) {
+                        std::printf("experts %d slots %d: tile at %d + %d of %d\n", n_exp, nslots, t.blk0, t.nblk, cap);
+                        return 1;
+                    }
+                    if (!wild && (!ok || t.blk0 != first + blocks || t.m0 != 16 * blocks)) return 2;
+                    blocks += t.nblk;
+                    slots += t.cnt;
+                }
+                if (!wild && (blocks != nb || slots != count[e])) return 3;
+                first += nb;
+                tiles += nt;
+            }
+            if (!wild && tiles > (mb == 1 ? cap : vb::moe_wreg_tiles(nslots, n_exp, mb))) return 4;
+        }
+    }
+    return 0;
+}
+"""
+
 
 def _run(tmp_path, code):
     cxx = shutil.which("g++") or shutil.which("clang++")
@@ -57,3 +103,9 @@ def _run(tmp_path, code):
 def test_rows_fetch_stays_inside(tmp_path):
     """Row groups of gemm_rows.hip: no load behind a ragged last group."""
     _run(tmp_path, ROWS)
+
+
+def test_moe_tiles_stay_inside(tmp_path):
+    """Expert tiles of moe_wreg.hip: any routing's tiles are all there, and
+    none of overwritten lists lies past the packed blocks."""
+    _run(tmp_path, MOE)

@@ -13,6 +13,7 @@
 // finds its (expert, tile) from the slot offsets with one wave scan;
 // workgroups past the last tile end at once.
 #include "mfma_q4k.hpp"
+#include "tile_index.hpp"
 #include "wreg_core.hpp"
 #include "vb_internal.hpp"
 #include "../../include/vbhip.h"
@@ -27,16 +28,10 @@ struct WregExperts {
     const uint8_t* p[MOE_KQ_MAX_EXPERTS];
 };
 
-struct Tile {
-    int e;        // expert
-    int blk0;     // first packed block (of all experts' blocks)
-    int nblk;     // blocks, 1 .. MB_MAX
-    int m0, cnt;  // first of the expert's slots, slots in the tile
-};
-
 // Work item `lin` of the routing's tiles x ncol column tiles (n_exp <= 64
 // experts, lane e = expert e): false past the last one, else the row tile and
-// its column tile.  Workgroups go to the eight XCDs round robin (lin % 8);
+// its column tile.  A tile past the packed blocks is dropped (moe_wreg_tile).
+// Workgroups go to the eight XCDs round robin (lin % 8);
 // each XCD takes a contiguous eighth of the tile-major order, so a tile's
 // packed rows are read into one or two XCDs' L2 only (down product at 8
 // experts, 125 slots each, 4096 x 14336: the rows dealt over all XCDs ran
@@ -44,7 +39,7 @@ struct Tile {
 // single blocks in order (the pack pass).
 template <int UNIT>
 __device__ __forceinline__ bool find_tile(const int32_t* __restrict__ eoff, const int32_t* __restrict__ elist,
-                                          int n_exp, int nslots, int lin, int ncol, Tile& t, int& col) {
+                                          int n_exp, int nslots, int lin, int ncol, MoeTile& t, int& col) {
     const int lane = static_cast<int>(threadIdx.x) & 63;
     const int c = lane < n_exp ? expert_slots(eoff, elist, lane < n_exp ? lane : 0, nslots).count : 0;
     const int nb = (c + 15) >> 4;
@@ -70,16 +65,9 @@ __device__ __forceinline__ bool find_tile(const int32_t* __restrict__ eoff, cons
     const uint64_t hit = __ballot(y >= st - nt && y < st);
     if (hit == 0) return false;
     const int e = __builtin_ctzll(hit);
-    const int ti = y - __builtin_amdgcn_readlane(st - nt, e);
-    const int nbe = __builtin_amdgcn_readlane(nb, e), nte = __builtin_amdgcn_readlane(nt, e);
-    const int bpt = UNIT == 1 ? 1 : (nbe + nte - 1) / nte;
-    const int bb = ti * bpt, ce = __builtin_amdgcn_readlane(c, e);
-    t.e = e;
-    t.blk0 = __builtin_amdgcn_readlane(sb - nb, e) + bb;
-    t.nblk = nbe - bb < bpt ? nbe - bb : bpt;
-    t.m0 = 16 * bb;
-    t.cnt = ce - t.m0 < 16 * t.nblk ? ce - t.m0 : 16 * t.nblk;
-    return true;
+    return moe_wreg_tile(e, y - __builtin_amdgcn_readlane(st - nt, e), __builtin_amdgcn_readlane(c, e),
+                         __builtin_amdgcn_readlane(sb - nb, e), UNIT == 1 ? 1 : MB_MAX,
+                         moe_wreg_blocks(nslots, n_exp), t);
 }
 
 // Packed activations: grid (blocks, h / 256), one 16 x 256 block each; rows
@@ -88,7 +76,7 @@ __device__ __forceinline__ bool find_tile(const int32_t* __restrict__ eoff, cons
 __global__ void __launch_bounds__(256) moe_wreg_pack(const _Float16* __restrict__ xh, const int32_t* __restrict__ eoff,
                                                      const int32_t* __restrict__ elist, int n_exp, int nslots, int topk,
                                                      int h, int q6, uint4* __restrict__ xf) {
-    Tile t;
+    MoeTile t;
     int col;
     if (!find_tile<1>(eoff, elist, n_exp, nslots, static_cast<int>(blockIdx.x), 1, t, col)) return;
     const SlotRange slots = expert_slots(eoff, elist, t.e, nslots);
@@ -113,7 +101,7 @@ __global__ void __launch_bounds__(256) moe_wreg_pack(const _Float16* __restrict_
 // and the same 16 up rows.
 template <int TYPE, int MB>
 __device__ __forceinline__ void gate_up_body(const uint8_t* wg, const uint8_t* wu, uint32_t wbytes, const uint8_t* xf,
-                                             const Tile& t, int h, int i_dim, uint32_t rb, int n0,
+                                             const MoeTile& t, int h, int i_dim, uint32_t rb, int n0,
                                              int q6_out, _Float16* __restrict__ hf, u32x4* b0, u32x4* b1) {
     const int lane = static_cast<int>(threadIdx.x) & 63, j = lane & 15, g = lane >> 4;
     const int wn = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -154,7 +142,7 @@ __global__ void __launch_bounds__(256, 2) moe_wreg_gate_up(WregExperts wg, WregE
                                                            _Float16* __restrict__ hf) {
     __shared__ u32x4 b0[BUF_U4];
     __shared__ u32x4 b1[BUF_U4];
-    Tile t;
+    MoeTile t;
     int col;
     if (!find_tile<MB_MAX>(eoff, elist, n_exp, nslots, static_cast<int>(blockIdx.x), i_dim / 64, t, col)) return;
     const int n0 = col * 64;
@@ -184,7 +172,7 @@ __global__ void __launch_bounds__(256, 2) moe_wreg_gate_up(WregExperts wg, WregE
 // exchange one column fragment's sums through LDS.
 template <int TYPE, int MB>
 __device__ __forceinline__ void down_body(const uint8_t* wd, uint32_t wbytes, const uint8_t* hf, const SlotRange& slots,
-                                          const Tile& t, int h, int i_dim, uint32_t rb, int n0, float* __restrict__ obuf,
+                                          const MoeTile& t, int h, int i_dim, uint32_t rb, int n0, float* __restrict__ obuf,
                                           const float* __restrict__ rw, int topk, float* __restrict__ yacc, u32x4* b0,
                                           u32x4* b1) {
     const int lane = static_cast<int>(threadIdx.x) & 63, j = lane & 15, g = lane >> 4;
@@ -234,7 +222,7 @@ __global__ void __launch_bounds__(512) moe_wreg_down(WregExperts wd, uint32_t wb
                                                      const float* __restrict__ rw, int topk, float* __restrict__ yacc) {
     __shared__ u32x4 b0[2 * BUF_U4];
     __shared__ u32x4 b1[2 * BUF_U4];
-    Tile t;
+    MoeTile t;
     int col;
     if (!find_tile<MB_MAX>(eoff, elist, n_exp, nslots, static_cast<int>(blockIdx.x), h / 128, t, col)) return;
     const SlotRange slots = expert_slots(eoff, elist, t.e, nslots);
@@ -272,10 +260,7 @@ bool moe_wreg_type(int32_t t) { return t == TYPE_Q4_K || t == TYPE_Q5_K || t == 
 int moe_wreg(int32_t gu_type, int32_t dn_type, const void* const* wg, const void* const* wu, const void* const* wd,
              int n_exp, const _Float16* xh, int nslots, int topk, int64_t h, int64_t i, const int32_t* eoff,
              const int32_t* elist, void* xf, void* hf, float* obuf, const float* rw, float* yacc, hipStream_t st) {
-    // most blocks (tiles) of any routing: every expert but one may leave a
-    // block (tile) partly filled
-    const int live = n_exp < nslots ? n_exp : nslots;
-    const int blocks = nslots / 16 + live, tiles = nslots / (16 * MB_MAX) + live;
+    const int blocks = moe_wreg_blocks(nslots, n_exp), tiles = moe_wreg_tiles(nslots, n_exp, MB_MAX);
     const int ih = static_cast<int>(h), ii = static_cast<int>(i);
     const uint32_t rb_gu = static_cast<uint32_t>(row_bytes(gu_type, h)), rb_d = static_cast<uint32_t>(row_bytes(dn_type, i));
     const uint32_t wb_gu = static_cast<uint32_t>((i * rb_gu + 3) & ~int64_t(3));

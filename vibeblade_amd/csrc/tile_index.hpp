@@ -20,4 +20,36 @@ constexpr uint32_t rows_fetch_at(int grp, int ngroups, uint32_t slot, uint32_t r
     return grp < ngroups && slot < rb ? (static_cast<uint32_t>(grp) * rb + slot) * 16u : ROWS_NONE;
 }
 
+// ---- expert tiles (moe_wreg.hip) -------------------------------------------------
+
+// Most 16-row blocks, and most tiles of up to `mb_max` blocks, that any
+// routing of `nslots` slots over `n_exp` experts makes: every expert with
+// slots may leave one partly filled.
+constexpr int moe_wreg_blocks(int nslots, int n_exp) { return nslots / 16 + (n_exp < nslots ? n_exp : nslots); }
+constexpr int moe_wreg_tiles(int nslots, int n_exp, int mb_max) {
+    return nslots / (16 * mb_max) + (n_exp < nslots ? n_exp : nslots);
+}
+
+struct MoeTile {
+    int e;        // expert
+    int blk0;     // first packed block (of all experts' blocks)
+    int nblk;     // blocks, 1 .. mb_max
+    int m0, cnt;  // first of the expert's slots, slots in the tile
+};
+
+// Tile `ti` of expert e with `slots` slots, whose blocks start at `first` of
+// all experts' and fill tiles of up to mb_max blocks (equal sizes).  False if
+// the tile's blocks do not all lie below `cap`: never so for lists the
+// routing wrote, but lists that another stream overwrote can claim more slots
+// than there are, and the packed and hidden rows hold `cap` blocks.
+constexpr bool moe_wreg_tile(int e, int ti, int slots, int first, int mb_max, int cap, MoeTile& t) {
+    const int nb = (slots + 15) / 16, nt = (nb + mb_max - 1) / mb_max, bpt = (nb + nt - 1) / nt, bb = ti * bpt;
+    t.e = e;
+    t.blk0 = first + bb;
+    t.nblk = nb - bb < bpt ? nb - bb : bpt;
+    t.m0 = 16 * bb;
+    t.cnt = slots - t.m0 < 16 * t.nblk ? slots - t.m0 : 16 * t.nblk;
+    return t.nblk > 0 && t.blk0 + t.nblk <= cap;
+}
+
 }  // namespace vb
