@@ -53,6 +53,14 @@ static int next(int n) { rnd = rnd * 1664525u + 1013904223u; return int((rnd >> 
 // each within [0, nslots] but of any sum, as overwritten lists can hold:
 // every accepted tile stays below moe_wreg_blocks.
 int main() {
+    // the rows fit from 16 slots per expert (where moe_wreg_shape begins), not
+    // from 14 (15 n_exp rows of padding)
+    for (int e = 1; e <= 64; e++)
+        for (int n = 1; n <= 1024; n++) {
+            const bool fits = vb::moe_wreg_fits(n, e);
+            if ((n >= 16 * e && !fits) || (n % 16 == 0 && n <= 14 * e && fits)) return 5;
+            if (fits && 16 * vb::moe_wreg_blocks(n, e) > 2 * n) return 6;
+        }
     for (int rep = 0; rep < 20000; rep++) {
         const int n_exp = 1 + next(64), nslots = 1 + next(1024), cap = vb::moe_wreg_blocks(nslots, n_exp);
         const bool wild = rep & 1;

@@ -24,6 +24,7 @@
 // Each expert's weights are streamed once per 16 routed slots.
 #include "mfma_q4k.hpp"
 #include "skinny_core.hpp"
+#include "tile_index.hpp"
 #include "vb_internal.hpp"
 #include "../../include/vbhip.h"
 
@@ -505,9 +506,11 @@ __global__ void __launch_bounds__(256) moe_combine_routed(const float* __restric
     *reinterpret_cast<float4*>(y + static_cast<int64_t>(t) * h + o) = s;
 }
 
-// Workspace: hbuf (slots x i, fp32 for F32 experts, fp16 for Q4_K), obuf
-// (slots x h fp32); Q4_K only: xh (tokens x h fp16), routing (ridx, rw),
-// per-expert slot lists (eoff, elist).
+// Workspace: hbuf (slots x i fp32: fp32 rows of F32 experts, fp16 rows of the
+// others, which moe_wreg.hip pads to blocks of 16: moe_wreg_fits), obuf (slots
+// x h fp32; before the down product moe_wreg.hip's packed fp16 activations,
+// padded likewise), xh (tokens x h fp16), routing (ridx, rw), per-expert slot
+// lists (eoff, elist).
 struct MoeWs {
     size_t hbuf, obuf, xh, ridx, rw, eoff, elist, total;
 };
@@ -630,10 +633,9 @@ extern "C" int vb_moe_grouped_ffn_types(const void* const* wg, const void* const
         // expert-grouped K-split kernel (gemm_kq.hip), gate/up with the same
         // SwiGLU epilogue
         const bool wreg = moe_wreg_type(gate_up_type) && moe_wreg_type(down_type) &&
-                          moe_wreg_shape(slots, n_exp, h);
+                          moe_wreg_shape(slots, n_exp, h) && moe_wreg_fits(static_cast<int>(slots), n_exp);
         if (wreg) {
-            // the packed rows (at most slots + 15 n_exp <= 2 slots of them)
-            // take obuf's place until the down product writes it
+            // the packed rows take obuf's place until the down product writes it
             rc = moe_wreg(gate_up_type, down_type, wg, wu, wd, n_exp, xh, static_cast<int>(slots), topk, h, i, eoff,
                           elist, obuf, hb16, obuf, rw, yacc, st);
             if (rc != OK) return rc;

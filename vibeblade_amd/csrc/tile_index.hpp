@@ -30,6 +30,12 @@ constexpr int moe_wreg_tiles(int nslots, int n_exp, int mb_max) {
     return nslots / (16 * mb_max) + (n_exp < nslots ? n_exp : nslots);
 }
 
+// Whether the blocks' fp16 rows fit where moe_ws (moe.hip) lays fp32 rows of
+// the slots: packed activations in obuf, hidden rows in hbuf.
+constexpr bool moe_wreg_fits(int nslots, int n_exp) {
+    return 16 * moe_wreg_blocks(nslots, n_exp) * 2 <= nslots * 4;
+}
+
 struct MoeTile {
     int e;        // expert
     int blk0;     // first packed block (of all experts' blocks)
