@@ -906,3 +906,21 @@ def test_rows(knob, qtype, m, n, k):
         y = gemm(qt, xt).cpu().numpy()
         assert np.all(np.isfinite(y))
         assert O.rel_l2(y, ref_gemm(qt, xt.float().cpu().numpy())) <= TOL, dtype
+
+
+@pytest.mark.parametrize("qtype,m,n,k,dtype", [(Q4K, 101, 1001, 8192, torch.float16),
+                                               (Q6K, 33, 301, 14336, torch.float32),
+                                               (Q4K, 601, 1001, 4096, torch.float32)])
+def test_split_sum_alignment(qtype, m, n, k, dtype):
+    """K splits summed (gemm_ksum) into an output that starts 4, 8 or 12 bytes
+    off a 16-byte boundary, with partial products of an odd number of values:
+    the bits of the aligned call, and nothing written beside them."""
+    qt, x = make(m, n, k, m + n, qtype=qtype)
+    xt = torch.from_numpy(x).to("cuda", dtype)
+    want = gemm(qt, xt)
+    assert O.rel_l2(want.cpu().numpy(), ref_gemm(qt, xt.float().cpu().numpy())) <= TOL
+    for off in (1, 2, 3):
+        buf = torch.full((m * n + 8,), 7.0, dtype=torch.float32, device="cuda")
+        gemm(qt, xt, out=buf[off:off + m * n].view(m, n))
+        assert torch.equal(buf[off:off + m * n].view(m, n), want)
+        assert torch.all(buf[:off] == 7.0) and torch.all(buf[off + m * n:] == 7.0)

@@ -509,17 +509,17 @@ __global__ void __launch_bounds__(XR_THREADS) gemm_xr_kernel(const uint8_t* __re
 }
 
 // Y = sum of the KS partial products in the order kz = 0, 1, ... (fixed,
-// deterministic); four outputs per thread.
+// deterministic); four outputs per thread.  Y may start at any float, and so
+// do the partial products after the first when M N is no multiple of 4: the
+// 16-byte accesses claim 4-byte alignment (one instruction all the same).
+typedef float float4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 __global__ void __launch_bounds__(256) xr_ksum_kernel(const float* __restrict__ P, float* __restrict__ Y,
                                                       int64_t total, int ks) {
     const int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
     if (i + 4 <= total) {
-        float4 s = *reinterpret_cast<const float4*>(P + i);
-        for (int z = 1; z < ks; z++) {
-            const float4 v = *reinterpret_cast<const float4*>(P + static_cast<int64_t>(z) * total + i);
-            s.x += v.x; s.y += v.y; s.z += v.z; s.w += v.w;
-        }
-        *reinterpret_cast<float4*>(Y + i) = s;
+        float4_t s = *reinterpret_cast<const float4_a4*>(P + i);
+        for (int z = 1; z < ks; z++) s += *reinterpret_cast<const float4_a4*>(P + static_cast<int64_t>(z) * total + i);
+        *reinterpret_cast<float4_a4*>(Y + i) = s;
     } else {
         for (int64_t e = i; e < total; e++) {
             float s = P[e];
