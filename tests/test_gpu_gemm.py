@@ -924,3 +924,32 @@ def test_split_sum_alignment(qtype, m, n, k, dtype):
         gemm(qt, xt, out=buf[off:off + m * n].view(m, n))
         assert torch.equal(buf[off:off + m * n].view(m, n), want)
         assert torch.all(buf[:off] == 7.0) and torch.all(buf[off + m * n:] == 7.0)
+
+
+@pytest.mark.parametrize("qtype,m,n,k,dtype", [(Q4K, 100, 300, 14336, torch.float16),
+                                               (ggml.GGML_TYPE_Q5_0, 300, 520, 15872, torch.float32)])
+def test_no_room_for_scratch(monkeypatch, qtype, m, n, k, dtype):
+    """Where the scratch of the faster kernels cannot be allocated, gemm()
+    runs the ones that do with less (nothing; the fp16 decode of the weights)."""
+    lib = _lib.load()
+    qt = make_other(qtype, n, k, m + n)
+    x = make(m, 1, k, m)[1]
+    xt = torch.from_numpy(x).to("cuda", dtype)
+    xdt = 1 if dtype == torch.float16 else 0
+    nb = lib.vb_gemm_scratch(m, n, k, qtype, xdt, 0)
+    need = lib.vb_gemm_workspace(m, n, k, qtype, xdt, 0)
+    assert 0 <= need < nb
+    want = gemm(qt, xt).cpu().numpy()
+    real, refused = torch.empty, []
+
+    def empty(*size, **kw):
+        if size == (nb,):
+            refused.append(nb)
+            raise torch.OutOfMemoryError("no room")
+        return real(*size, **kw)
+    monkeypatch.setattr(torch, "empty", empty)
+    y = gemm(qt, xt)
+    monkeypatch.undo()
+    assert refused == [nb]
+    # the same fp16 operands in another order of fp32 sums
+    assert O.rel_l2(y.cpu().numpy(), want) <= 1e-5

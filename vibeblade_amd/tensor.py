@@ -171,10 +171,18 @@ def gemm(w: QTensor, x: torch.Tensor, out: torch.Tensor | None = None,
     lib = _lib.load()
     nb = int(lib.vb_gemm_scratch(m, w.rows, w.k, w.qtype, xdt, variant))
     if nb > 0:
-        # packed X and partial products, from torch's caching allocator
-        ws = torch.empty(nb, dtype=torch.uint8, device=w.device)
+        # packed X and partial products, from torch's caching allocator; with
+        # no room for them what the call cannot do without (vb_gemm_ws then
+        # runs the kernels that fit)
+        try:
+            ws = torch.empty(nb, dtype=torch.uint8, device=w.device)
+        except torch.OutOfMemoryError:
+            need = int(lib.vb_gemm_workspace(m, w.rows, w.k, w.qtype, xdt, variant))
+            if need >= nb:
+                raise
+            nb, ws = need, (torch.empty(need, dtype=torch.uint8, device=w.device) if need > 0 else None)
         _lib.call("vb_gemm_ws", w.ptr(), x.data_ptr(), xdt, out.data_ptr(), m, w.rows, w.k, w.qtype,
-                  variant, ws.data_ptr(), nb, _stream())
+                  variant, ws.data_ptr() if ws is not None else None, nb, _stream())
         return out
     _lib.call("vb_gemm", w.ptr(), x.data_ptr(), xdt, out.data_ptr(), m, w.rows, w.k, w.qtype,
               variant, _stream())
