@@ -42,6 +42,27 @@ int main() {
 }
 """
 
+PITCH = r"""
+#include <cstdio>
+#include <initializer_list>
+#include "tile_index.hpp"
+// Q5_K and Q8_0 rows of up to 16 super-blocks: the same offset of 16 rows in
+// 16 different slots of a bank round, and the image in its 16 rows + 32 slots
+int main() {
+    for (uint32_t block : {176u, 272u})
+        for (uint32_t nsb = 1; nsb <= 16; nsb++) {
+            const uint32_t rb = block * nsb, pitch = vb::rows_pitch(rb);
+            uint32_t banks = 0;
+            for (uint32_t j = 0; j < 16; j++) banks |= 1u << (j * pitch / 16 % 16);
+            if (pitch % 16 != 0 || pitch < rb || banks != 0xFFFFu || 16 * pitch > 16 * (16 * block + 32) - 16) {
+                std::printf("rows of %u bytes: pitch %u\n", rb, pitch);
+                return 1;
+            }
+        }
+    return 0;
+}
+"""
+
 MOE = r"""
 #include <cstdio>
 #include <initializer_list>
@@ -111,6 +132,11 @@ def _run(tmp_path, code):
 def test_rows_fetch_stays_inside(tmp_path):
     """Row groups of gemm_rows.hip: no load behind a ragged last group."""
     _run(tmp_path, ROWS)
+
+
+def test_rows_image_spreads_over_banks(tmp_path):
+    """Row images of gemm_rows.hip: no two rows of a read on the same banks."""
+    _run(tmp_path, PITCH)
 
 
 def test_moe_tiles_stay_inside(tmp_path):

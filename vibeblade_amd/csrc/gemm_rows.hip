@@ -52,11 +52,11 @@ __global__ void __launch_bounds__(64 * ROWS_WAVES) gemm_rows_kernel(const uint8_
                                                                     const void* __restrict__ X, float* __restrict__ Y,
                                                                     int M, int N, int K, uint32_t rb) {
     using T = Kq<TYPE>;
-    // Rows a multiple of 256 bytes long put the 16 rows of a read on the same
-    // banks: a 16-byte gap after each (Q8_0 14336 x 4096: 29 us without, 19
-    // with).  Q6_K rows (210 bytes a block) spread by themselves and need not
-    // be whole slots.
-    constexpr bool GAP = TYPE != TYPE_Q6_K;
+    // Rows of an even number of 16-byte slots put the 16 rows of a read on few
+    // banks and get a slot's gap (rows_pitch; Q8_0 14336 x 4096: 29 us without,
+    // 19 with).  Q6_K rows (210 bytes a block) spread by themselves and need
+    // not be whole slots.
+    constexpr bool WHOLE = TYPE != TYPE_Q6_K;
     constexpr int P = rows_pieces(TYPE), IMG = 16 * rows_block_bytes(TYPE) + 32;  // 16-byte slots
     __shared__ u32x4 b0[IMG];
     __shared__ u32x4 b1[IMG];
@@ -71,12 +71,13 @@ __global__ void __launch_bounds__(64 * ROWS_WAVES) gemm_rows_kernel(const uint8_
 
     // rows 16 grp .. + 15; rows and groups past the last read nothing
     u32x4 st[P];
-    const uint32_t pitch = rb + (GAP ? 16u : 0u);
+    const uint32_t pitch = WHOLE ? rows_pitch(rb) : rb;
+    const uint32_t gap = (pitch - rb) >> 4;
     int at[P];  // the lane's slots in an image; pieces past the rows go to its last one
 #pragma unroll
     for (int i = 0; i < P; i++) {
         const uint32_t slot = static_cast<uint32_t>((wave + ROWS_WAVES * i) * 64 + lane);
-        at[i] = slot < rb ? static_cast<int>(slot + (GAP ? slot / (rb >> 4) : 0u)) : IMG - 1;
+        at[i] = slot < rb ? static_cast<int>(slot + (WHOLE ? slot / (rb >> 4) * gap : 0u)) : IMG - 1;
     }
     auto fetch = [&](int grp) __attribute__((always_inline)) {
 #pragma unroll

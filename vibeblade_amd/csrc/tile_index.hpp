@@ -20,6 +20,12 @@ constexpr uint32_t rows_fetch_at(int grp, int ngroups, uint32_t slot, uint32_t r
     return grp < ngroups && slot < rb ? (static_cast<uint32_t>(grp) * rb + slot) * 16u : ROWS_NONE;
 }
 
+// Bytes from one row to the next in the LDS image, for rows of whole 16-byte
+// slots.  The 16 rows that a read touches at the same offset fall on distinct
+// banks when a row is an odd number of slots (64 banks of 4 bytes: 16 slots a
+// round); a row of an even number gets one more.
+constexpr uint32_t rows_pitch(uint32_t rb) { return rb | 16u; }
+
 // ---- expert tiles (moe_wreg.hip) -------------------------------------------------
 
 // Most 16-row blocks, and most tiles of up to `mb_max` blocks, that any
