@@ -146,9 +146,11 @@ int vb_gemv(const void* w, const float* x, float* y, int64_t n, int64_t k,
  * 33 <= m <= 64 and (k >= 8192) 2 <= m <= 16; 3 at 257 <= m <= 768 for fp16
  * X and n >= 8192.  Q6_K / Q8_0: 4 up to m = 64 (at n < 8192: Q6_K up to
  * m = 256 with fp16 X, both up to 128 with fp32 X), 2 above.  Q5_K: 4 up to
- * m = 32 (64 at n < 8192), 2 above.  At 2 <= m <= 16 and k <= 4096 Q5_K (n >=
- * 2048), Q6_K and Q8_0 (n >= 10240) stream whole weight rows instead
- * (gemm_rows.hip).  Variants 1 and 3 are Q4_K-only.  With variant 0 and
+ * m = 32 (64 at n < 8192), 2 above.  At 2 <= m <= 16 and
+ * 1024 <= k <= 4096, k % 256 == 0, Q5_K (n > 8192; n >= 2048 at k = 2048 and
+ * 4096; n >= 16384 below k = 2048), Q6_K (n >= 10240; n >= 24576 below k =
+ * 1536) and Q8_0 (n >= 10240; n > 16384 below k = 2048, n >= 24576 below
+ * 1536) stream whole weight rows instead (gemm_rows.hip).  Variants 1 and 3 are Q4_K-only.  With variant 0 and
  * m == 1 the GEMV runs instead: vb_gemv's kernels for fp32 X (bit-identical
  * to vb_gemv), and for fp16 X the short-row kernels reading the halves
  * directly (Q4_K k <= 4096; Q6_K k = 2048 / 4096; Q8_0 k % 256 == 0 up to

@@ -63,6 +63,28 @@ int main() {
 }
 """
 
+RULE = r"""
+#include <cstdio>
+#include <initializer_list>
+#include "tile_index.hpp"
+// calls that ran slower on the row-streaming kernel stay off it, calls that
+// gained stay on it
+struct Call { bool q5k, q8; int64_t n, k; bool on; };
+int main() {
+    for (Call c : {Call{true, false, 8192, 2560, false}, Call{true, false, 4096, 3584, false},
+                   Call{true, false, 2048, 3072, false}, Call{true, false, 8192, 3072, false},
+                   Call{false, true, 14336, 1536, false}, Call{false, true, 12606, 1792, false},
+                   Call{false, false, 128256, 4096, true}, Call{false, true, 14336, 4096, true},
+                   Call{true, false, 2048, 4096, true}, Call{true, false, 14336, 3072, true},
+                   Call{false, false, 10240, 2048, true}, Call{false, true, 24576, 1536, true}})
+        if (vb::rows_lead(c.q5k, c.q8, c.n, c.k) != c.on) {
+            std::printf("%lld x %lld\n", (long long)c.n, (long long)c.k);
+            return 1;
+        }
+    return 0;
+}
+"""
+
 MOE = r"""
 #include <cstdio>
 #include <initializer_list>
@@ -137,6 +159,11 @@ def test_rows_fetch_stays_inside(tmp_path):
 def test_rows_image_spreads_over_banks(tmp_path):
     """Row images of gemm_rows.hip: no two rows of a read on the same banks."""
     _run(tmp_path, PITCH)
+
+
+def test_rows_rule(tmp_path):
+    """Which calls gemm_rows.hip takes: none of those that lost time on it."""
+    _run(tmp_path, RULE)
 
 
 def test_moe_tiles_stay_inside(tmp_path):

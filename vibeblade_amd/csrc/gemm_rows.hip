@@ -157,21 +157,12 @@ __global__ void __launch_bounds__(64 * ROWS_WAVES) gemm_rows_kernel(const uint8_
 
 }  // namespace
 
-// Where the row groups are enough to stream.  MI355X, us K-split kernel / this
-// one, fp16 X, M = 2 and 16:
-//   Q5_K 14336x4096  26.8 / 17.9  31.7 / 19.9    Q6_K 14336x4096  23.3 / 17.6  27.2 / 20.1
-//   Q5_K 4096x4096   10.2 / 8.6   12.5 / 10.9    Q6_K 10240x4096  21.9 / 15.3  25.9 / 17.4
-//   Q5_K 2048x2048    7.4 / 5.9    8.7 / 7.0     Q6_K 8192x4096   12.3 / 13.0  13.5 / 14.9
-//   Q5_K 4096x1536    5.2 / 5.9    5.5 / 6.8     Q6_K 11000x2048  12.7 / 10.7  14.0 / 11.9
-//   Q5_K 16384x1024   9.3 / 8.7    9.8 / 9.6     Q6_K 4096x4096    8.1 / 8.5   10.2 / 10.8
-//   Q8_0 14336x4096  26.5 / 19.0  33.0 / 21.8    Q8_0 28672x1024  15.0 / 14.5  16.6 / 15.5
-//   Q8_0 24576x1536  20.8 / 15.8  22.9 / 16.6    Q8_0 16384x1024   8.7 / 10.5   9.0 / 11.1
+// The rule and what it was measured on: rows_lead (tile_index.hpp).
 bool gemm_rows_shape(int32_t type, int64_t M, int64_t N, int64_t K) {
     if (type != TYPE_Q5_K && type != TYPE_Q6_K && type != TYPE_Q8_0) return false;
     if (M < 2 || M > 16 || K % 256 != 0 || K > ROWS_MAX_K || N * row_bytes(type, K) >= (int64_t(1) << 31)) return false;
     if (knobs().gemm_rows_min_n >= 0) return N >= knobs().gemm_rows_min_n;
-    if (type == TYPE_Q5_K) return K >= 2048 ? N >= 2048 : K >= 1024 && N >= 16384;
-    return K >= 1536 ? N >= 10240 : K >= 1024 && N >= 24576;
+    return rows_lead(type == TYPE_Q5_K, type == TYPE_Q8_0, N, K);
 }
 
 int gemm_rows(const void* w, const void* X, int32_t x_dtype, float* Y, int64_t M, int64_t N, int64_t K, int32_t type,

@@ -26,6 +26,27 @@ constexpr uint32_t rows_fetch_at(int grp, int ngroups, uint32_t slot, uint32_t r
 // round); a row of an even number gets one more.
 constexpr uint32_t rows_pitch(uint32_t rb) { return rb | 16u; }
 
+// Where that kernel leads the K-split kernel, at every number of rows from 2 to
+// 16 and for both types of X.  MI355X, K-split over row-streaming time, the
+// least over those rows at the shapes measured:
+//   Q5_K      K = 2048, 4096   other K >= 2048      1024 <= K < 2048
+//     N <=  4096     1.15 - 1.18      0.87 - 0.94           -
+//     N <=  8192     1.21 - 1.61      0.86 - 1.15           -
+//     N <= 16384     1.60 - 1.88      1.00 - 1.30           -
+//     above          1.91 - 2.46      1.41 - 1.94      1.20 - 1.64
+//   K >= 2048, N 10240 .. 16384 and above: Q6_K 1.09 - 1.59, 1.48 - 2.07; Q8_0
+//     1.03 - 1.70, 1.48 - 2.19
+//   1536 <= K < 2048: Q6_K 0.98 - 1.19, 1.29 - 1.56; Q8_0 0.92 - 1.12, 1.33 - 1.60
+//   1024 <= K < 1536, N >= 24576: Q6_K 1.18 - 1.57, Q8_0 1.08 - 1.33
+// (a wave owns an eighth of K in steps of 128, so only multiples of 1024 give
+// the waves equal work, and up to N = 8192 a workgroup has two groups at most
+// to make up for its first loads)
+constexpr bool rows_lead(bool q5k, bool q8, int64_t N, int64_t K) {
+    if (K < 1024) return false;
+    if (q5k) return K >= 2048 ? N > 8192 || (N >= 2048 && K % 2048 == 0) : N >= 16384;
+    return K >= 2048 ? N >= 10240 : (K >= 1536 ? N >= (q8 ? 16385 : 10240) : N >= 24576);
+}
+
 // ---- expert tiles (moe_wreg.hip) -------------------------------------------------
 
 // Most 16-row blocks, and most tiles of up to `mb_max` blocks, that any
