@@ -116,43 +116,111 @@ int64_t wreg_packed_bytes(int64_t M, int64_t K) { return (M + 15) / 16 * 16 * K 
 
 }  // namespace
 
-// Where this kernel leads.  MI355X, us old / this one (the packing and the
-// sum of the splits included), old = the skinny, K-split or tiled kernel:
-//   fp16 X            M = 17       32         64         128        256
-//   Q4_K 4096x14336   29.2 / 21.3  36 / 22    63 / 26    69 / 34    77 / 52
-//   Q6_K 4096x14336   29.7 / 27.5  39 / 28    62 / 32    90 / 42    87 / 70
-//   Q8_0 4096x14336   37.6 / 29.9             81 / 34    96 / 42    101 / 64
-//   Q4_K 8192x8192    19.7 / 21.9             36 / 24    51 / 34    84 / 55
-//   Q6_K 4096x8192    17.7 / 21.0             31 / 23    55 / 31    56 / 48
-//   Q4_K 4096x4096    11.5 / 13.9  14 / 15    21.3 / 17  24 / 20    26.6 / 27.2
-//   Q6_K 4096x4096    10.3 / 17.8  13 / 19    20.3 / 22  27 / 24    28 / 34
-//   Q4_K 14336x4096   13.3 / 19.6  16 / 21    26.2 / 24  33.1 / 33  54 / 52
-//   Q5_K 14336x4096   26.8 / 25.0             39 / 29    42 / 38    68.0 / 68.4
-//   Q4_K 32768x2048   16.7 / 18.2             26 / 21    42 / 32    66 / 51
-//   Q4_K 8192x2048     8.1 / 13.5             13.8 / 15  18 / 19    26.6 / 27.6
+// Where this kernel leads: the smallest K, in super-blocks, from which it does
+// at every K measured (0: not taken), by the rows of X (up to 32, 64, 128, 192,
+// 256) and the columns (N up to 511, 2047, 4096, 8191, 16384, 32768, more).
+//
+// Measured on MI355X over 68000 calls (each type and X; 11 to 19 values of M;
+// N from 16 to 151936, K from 2048 to 28672, on a grid and at random; weights
+// not in cache) against the skinny, K-split or tiled kernel that the call ran
+// on before, the packing and the sum of the splits included.  No call that the
+// table takes ran below 0.97 of the other kernel's rate; they gain 2.06 in the
+// geometric mean; the ones left out are 1.14 in the mean and 0.63 at the worst.
+// Some of both, us other / this one:
+//   fp16 X            M = 17       32           64           128          256
+//   Q4_K 4096x14336   29.5 / 21.9  35.2 / 22.3  62.8 / 25.8  77.3 / 33.8  78.7 / 49.2
+//   Q6_K 4096x14336   29.8 / 28.5  38.7 / 28.8  61.5 / 32.4  90.1 / 43.2  86.0 / 68.3
+//   Q8_0 8192x8192    43.6 / 30.3  56.0 / 29.7  89.8 / 33.1  58.1 / 41.3  74.1 / 63.5
+//   Q4_K 4096x4096                              21.6 / 17.4  23.6 / 20.4
+//   Q5_K 14336x4096   26.7 / 25.5  29.6 / 26.2  38.0 / 29.6  39.4 / 38.1  62.8 / 66.8
+//   Q5_K 32768x2048                             40.8 / 27.5  43.4 / 34.6  47.9 / 62.7
 //   fp32 X (the other kernels convert it in every column tile)
-//   Q4_K 4096x14336   44.6 / 21.6             87 / 24    84 / 34    96 / 53
-//   Q8_0 4096x14336   58.7 / 30.1            132 / 32   114 / 43   124 / 66
-//   Q4_K 4096x4096    16.2 / 13.9             29 / 16    29 / 23    31 / 27
-//   Q6_K 14336x4096   31.4 / 27.6             41 / 31    58 / 44    79 / 73
-// Below K = 4096 the three launches and the first loads cost more than the
-// decode saved, unless N is large.
+//   Q4_K 4096x14336   44.6 / 22.3  63.1 / 23.0  112 / 26.3   92.4 / 34.4  93.9 / 50.4
+//   Q4_K 14336x4096                             30.4 / 25.0  39.8 / 32.6  55.7 / 48.1
+//   Q6_K 4096x4096                              34.4 / 21.8  27.8 / 24.4  36.6 / 29.4
+// Why the lines lie there: the packing and the sum of the splits are launches
+// of their own, which a small K does not pay for; up to 64 rows with fp16 X the
+// other kernels decode a weight once as well; and above 192 rows the tiles of
+// 16 blocks spill 34 / 27 / 11 registers on Q5_K / Q6_K / Q8_0.
+constexpr uint8_t kWregMinSb[4][2][5][7] = {
+    {
+        { // Q4_K, X fp16
+            {32, 32, 32, 39,  0,  0,  0},
+            {32, 24, 24, 16,  0,  8,  0},
+            {32, 16, 16, 23, 16,  8,  8},
+            {32, 20, 21, 27, 16,  8,  8},
+            {32, 20, 39, 20, 21,  8, 10},
+        },
+        { // X fp32
+            {32, 16, 19, 16, 32,  0,  0},
+            {32, 16, 16, 16, 13,  8,  8},
+            {32, 16, 16, 16, 12,  8,  8},
+            {32, 16, 16, 16, 12,  8,  8},
+            {32, 16, 16, 16, 14,  8,  8},
+        },
+    },
+    {
+        { // Q5_K, X fp16
+            {48, 50, 52, 32, 21, 12,  0},
+            {32, 31, 32, 16, 12,  8,  8},
+            {32, 16, 16, 16, 14,  8,  8},
+            {32, 20, 20, 20, 13, 10,  8},
+            {32, 20, 30, 39,  0,  0,  0},
+        },
+        { // X fp32
+            {32, 32, 32, 32, 13, 12, 12},
+            {32, 16, 16, 16, 12,  8,  8},
+            {32, 16, 16, 16, 12,  8,  8},
+            {32, 16, 16, 16, 12,  8,  8},
+            {32, 16, 27, 16, 23,  0,  0},
+        },
+    },
+    {
+        { // Q6_K, X fp16
+            {48, 50, 52, 48, 48,  0,  0},
+            {32, 31, 32, 24, 24,  8,  0},
+            {32, 16, 16, 20, 16,  8,  8},
+            {32, 20, 20, 20, 20, 20, 20},
+            {32, 20, 32, 20, 25,  0,  0},
+        },
+        { // X fp32
+            {32, 32, 32, 32, 32,  0,  0},
+            {32, 16, 16, 16, 12,  8,  8},
+            {32, 16, 16, 16, 12,  8,  8},
+            {32, 16, 16, 16, 12,  8,  8},
+            {32, 16, 16, 16, 14,  0,  0},
+        },
+    },
+    {
+        { // Q8_0, X fp16
+            {48, 50, 47, 32, 14, 12, 16},
+            {32, 31, 30, 16, 13,  8, 10},
+            {32, 16, 16, 19, 14,  8,  8},
+            {32, 20, 20, 23, 14, 10, 10},
+            {32, 20, 30, 27, 25,  0,  0},
+        },
+        { // X fp32
+            {32, 32, 32, 32, 12, 12, 12},
+            {32, 16, 16, 16, 12,  8,  8},
+            {32, 16, 16, 16, 12,  8,  8},
+            {32, 16, 16, 20, 12,  8,  8},
+            {32, 16, 16, 16, 14,  0,  0},
+        },
+    },
+};
+
 bool gemm_wreg_shape(int32_t type, int32_t x_dtype, int64_t M, int64_t N, int64_t K) {
-    if (type != TYPE_Q4_K && type != TYPE_Q5_K && type != TYPE_Q6_K && type != TYPE_Q8_0) return false;
-    if (K % 256 != 0 || M < 2 || M > 16 * wreg::MB_MAX) return false;
+    const int t = type == TYPE_Q4_K ? 0 : (type == TYPE_Q5_K ? 1 : (type == TYPE_Q6_K ? 2 : (type == TYPE_Q8_0 ? 3 : -1)));
+    if (t < 0 || K % 256 != 0 || M < 2 || M > 16 * wreg::MB_MAX) return false;
     if (knobs().gemm_wreg_min_m >= 0) return M >= knobs().gemm_wreg_min_m;
-    const bool q6 = type == TYPE_Q6_K, f32 = x_dtype == X_F32, wide = N >= 8192;
-    const bool slow = type == TYPE_Q5_K || type == TYPE_Q8_0;  // no skinny kernel
-    if (M < 17) return f32 && K >= 12288 && !wide && M >= 8;
-    if (K >= 8192) return M > 32 || f32 || (q6 ? K >= 12288 : !(wide && type == TYPE_Q4_K));
-    if (N < 512) return false;  // one to four workgroups per K split
-    if (K >= 4096) {
-        if (M <= 32) return wide ? slow : f32 && type == TYPE_Q4_K;
-        if (M <= 64) return f32 || (N >= 1024 && (q6 ? K >= 6144 : !(wide && type == TYPE_Q4_K)));
-        return M <= 128 || f32 || K >= 5120 || (wide && !q6);
-    }
-    if (K >= 3072 && wide && (slow ? M > 16 : f32 && M > 32)) return true;
-    return M > 32 && K >= 2048 && N >= 16384 && (f32 || !q6 || M <= 128);
+    const bool f32 = x_dtype == X_F32;
+    // few rows: the conversion of fp32 X alone makes it worth it (M = 8, 4096 x
+    // 12288: Q4_K 25.9 / 20.5, Q8_0 32.0 / 28.2)
+    if (M < 17) return f32 && M >= 8 && N < 8192 && K >= (type == TYPE_Q6_K ? 14336 : 12288);
+    const int m = M <= 32 ? 0 : (M <= 64 ? 1 : (M <= 128 ? 2 : (M <= 192 ? 3 : 4)));
+    const int n = N <= 511 ? 0 : (N <= 2047 ? 1 : (N <= 4096 ? 2 : (N <= 8191 ? 3 : (N <= 16384 ? 4 : (N <= 32768 ? 5 : 6)))));
+    const int64_t sb = kWregMinSb[t][f32 ? 1 : 0][m][n];
+    return sb != 0 && K >= 256 * sb;
 }
 
 int64_t gemm_wreg_workspace(int64_t M, int64_t N, int64_t K) {
