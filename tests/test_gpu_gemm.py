@@ -864,7 +864,7 @@ def test_wreg(knob, qtype, m, n, k):
 @pytest.mark.parametrize("qtype,m,n,k,dtype", [(Q4K, 100, 1024, 14336, torch.float16),
                                                (Q6K, 33, 300, 8192, torch.float16),
                                                (Q80, 8, 300, 12288, torch.float32),
-                                               (Q6K, 300, 8200, 512, torch.float32),
+                                               (Q6K, 300, 14336, 512, torch.float32),
                                                (Q4K, 600, 1000, 4096, torch.float32)])
 def test_scratch_routes(qtype, m, n, k, dtype):
     """Routes that vb_gemm_scratch opens: the register-decoding kernel and

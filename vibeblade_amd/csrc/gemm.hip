@@ -748,20 +748,35 @@ int gemm_other(const void* w, const void* X, int32_t x_dtype, float* Y, int64_t 
 // The packed-X kernel beyond the shapes whose workspace vb_gemm_workspace
 // states, with the splits of gemm_xr_ksplit_even: fp32 X (the tiled kernel
 // converts it once per column tile), and fp16 X at N < 8192 for the types
-// whose other kernels decode slowly.  MI355X, us old / packed-X: fp32 X, Q6_K
-// 4096 x 14336 at M = 777 250 / 163, 14110 x 3072 at 359 125 / 61, Q4_K 14336
-// x 4096 at 512 94 / 64, 1773 x 13056 at 279 144 / 46, 4187 x 4864 at 828 69 /
-// 75, 1024 x 1024 at 300 16 / 22; fp16 X, Q4_0 5461 x 12288 at 533 229 / 131,
-// 5487 x 1536 at 972 53 / 35, 684 x 1536 at 414 16 / 26, Q5_K 7056 x 6400 at
-// 992 122 / 98, 2499 x 1792 at 941 33 / 33 (Q4_K, Q6_K and Q8_0 there keep
-// the tiled kernel: Q8_0 7943 x 8448 at 845 169 / 201).
+// whose other kernels decode slowly (Q4_K, Q6_K and Q8_0 keep the tiled kernel
+// there: Q8_0 7943 x 8448 at M = 845 169 us tiled / 201).  A short K does not
+// pay for the packing unless the rounds of workgroups fill the CUs (`busy`, in
+// percent); a long one mostly does in any case.  MI355X, 40000 calls timed (M
+// from 257 to 4096, K from 256 to 28672), rate against the kernel that the
+// call ran on before, the least and the geometric mean:
+//   fp32 X, the types but Q4_K   taken 0.92, 1.68 - 1.96   left out 0.55, 1.1 - 1.3
+//   fp32 X, Q4_K                 taken 0.93, 1.75          left out 0.68, 1.2
+//   fp16 X, Q4_0 / Q4_1          taken 0.89, 1.6           left out 0.70, 1.4
+//   fp16 X, Q5_K / Q5_0 / Q5_1   taken 0.93, 1.42 - 1.48   left out 0.65, 1.2 - 1.3
+// Some of them, us before / packed-X: fp32 X, Q6_K 4096 x 14336 at M = 777
+// 250 / 159, 3000 x 1536 at 300 17.6 / 28.0 (left out: 30 % busy), Q4_K 14336 x
+// 4096 at 512 94 / 64, 9871 x 4096 at 513 83 / 110 (left out: 52 % busy), Q8_0
+// 2048 x 2048 at 300 19.0 / 25.6 (left out: 30 %); fp16 X, Q4_0 5461 x 12288 at
+// 533 229 / 131, Q5_K 4096 x 5120 at 2048 95 / 130 (left out: 5 splits).
 static bool xr_even_shape(int32_t type, int32_t x_dtype, int64_t M, int64_t N, int64_t K) {
     if (!gemm_xr_type(type) || M <= 256 || M > INT32_MAX || K % 256 != 0) return false;
-    const bool b32 = gemm_b32_type(type);
-    if (!b32 && type != TYPE_Q4_K && type != TYPE_Q5_K && !knobs().gemm_xr_kq) return false;
-    if (x_dtype == X_F32) return N * K >= 4000000 && !(type == TYPE_Q4_K && N < 8192 && M > 768);
-    return N < 8192 && gemm_xr_ksplit(M, N, K) == 1 &&
-           ((b32 && N * K >= 8000000) || (type == TYPE_Q5_K && N * K >= 16000000));
+    const bool b32 = gemm_b32_type(type), q4k = type == TYPE_Q4_K;
+    if (!b32 && !q4k && type != TYPE_Q5_K && !knobs().gemm_xr_kq) return false;
+    const int ks = gemm_xr_ksplit_even(M, N, K), busy = gemm_xr_busy(M, N, ks);
+    if (x_dtype == X_F32) {
+        if (N * K < 4000000) return false;
+        if (q4k && N < 8192) return M <= 768 && (K >= 4096 || busy >= 90);
+        if (q4k) return busy >= 90 || (N > 16384 && K >= 2048);
+        return K >= 4096 || (N >= 8192 && K >= 2048) || busy >= (K >= 1024 ? 70 : 80);
+    }
+    if (N >= 8192 || gemm_xr_ksplit(M, N, K) > 1) return false;
+    if (b32 && !gemm_b32_high(type)) return N * K >= 8000000 && busy >= (M <= 1024 ? 80 : 90);
+    return (b32 || type == TYPE_Q5_K) && N * K >= (b32 ? 8000000 : 16000000) && busy >= 80 && ks <= 2;
 }
 
 int gemm_dispatch(const void* w, const void* X, int32_t x_dtype, float* Y, int64_t M, int64_t N, int64_t K,
