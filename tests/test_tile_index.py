@@ -112,7 +112,7 @@ int main() {
             count[e] = wild ? next(nslots + 1) : (e + 1 < n_exp ? next(left + 1) >> next(4) : left);
             if (!wild) left -= count[e];
         }
-        for (int mb : {1, 16}) {
+        for (int mb : {1, 10, 16}) {
             first = tiles = 0;
             for (int e = 0; e < n_exp; e++) {
                 const int nb = (count[e] + 15) / 16, nt = (nb + mb - 1) / mb;

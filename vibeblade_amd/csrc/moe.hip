@@ -36,7 +36,7 @@ constexpr int MOE_MAX_TOPK = 8;
 constexpr int MOE_MAX_SLOTS = 1024;  // tokens * topk
 
 // Whether the experts run on moe_wreg.hip, which decodes each weight once per
-// up to 256 slots but cannot fill the chip with a small down product (its
+// up to 160 slots but cannot fill the chip with a small down product (its
 // workgroups take 128 of the h columns of one expert).  MI355X, Q4_K gate/up
 // and Q6_K down, mean slots per expert in brackets: 8 experts of 4096 x 14336
 // 304 us against 307 at [12], 297 / 412 [16], 314 / 656 [32], 477 / 2168

@@ -1,5 +1,5 @@
 // Expert-grouped MoE products for prefill-sized batches: the weights of a hit
-// expert are read and decoded once per 256 of its slots (wreg_core.hpp), where
+// expert are read and decoded once per 160 of its slots (wreg_core.hpp), where
 // the skinny and K-split expert kernels (moe.hip, gemm_kq.hip) do so once per
 // 16.
 //
@@ -8,7 +8,7 @@
 // rows written straight in the down kernel's fragment order) and down.
 //
 // An expert's slots fill ceil(count / 16) blocks of 16 rows; its blocks make
-// ceil(blocks / 16) tiles of equal size.  The host knows only the slot count,
+// ceil(blocks / 10) tiles of equal size.  The host knows only the slot count,
 // so the grids hold the most tiles any routing can give, and every workgroup
 // finds its (expert, tile) from the slot offsets with one wave scan;
 // workgroups past the last tile end at once.
@@ -22,7 +22,15 @@ namespace vb {
 namespace {
 
 using wreg::BUF_U4;
-using wreg::MB_MAX;
+
+// Blocks per tile.  One kernel holds every tile height, so the tallest sets the
+// registers of all: bodies of 16 blocks spilled (14 / 46 / 63 / 42 registers in
+// gate/up on Q4_K / Q5_K / Q6_K / Q8_0, up to 42 in down), and one tall tile
+// left the CUs idle that two of half its height fill.  MI355X, 2 experts of
+// 4096 x 14336, slots each, us with tiles of up to 16 / 12 / 10 blocks: Q4_K
+// gate/up, Q6_K down 160 280 / 279 / 287, 192 319 / 324 / 281, 208 464 / 291 /
+// 290, 256 483 / 317 / 325, 512 627 / 494 / 449; Q8_0, Q5_K 208 547 / - / 313.
+constexpr int MB_MAX = 10;
 
 struct WregExperts {
     const uint8_t* p[MOE_KQ_MAX_EXPERTS];
@@ -159,10 +167,7 @@ __global__ void __launch_bounds__(256, 2) moe_wreg_gate_up(WregExperts wg, WregE
         case 7: VB_WREG_GU(7); break;
         case 8: VB_WREG_GU(8); break;
         case 9: VB_WREG_GU(9); break;
-        case 10: VB_WREG_GU(10); break;
-        case 11:
-        case 12: VB_WREG_GU(12); break;
-        default: VB_WREG_GU(16); break;
+        default: VB_WREG_GU(10); break;
     }
 #undef VB_WREG_GU
 }
@@ -239,10 +244,7 @@ __global__ void __launch_bounds__(512) moe_wreg_down(WregExperts wd, uint32_t wb
         case 7: VB_WREG_DN(7); break;
         case 8: VB_WREG_DN(8); break;
         case 9: VB_WREG_DN(9); break;
-        case 10: VB_WREG_DN(10); break;
-        case 11:
-        case 12: VB_WREG_DN(12); break;
-        default: VB_WREG_DN(16); break;
+        default: VB_WREG_DN(10); break;
     }
 #undef VB_WREG_DN
 }

@@ -192,7 +192,7 @@ int moe_kq(int32_t type, bool gate_up, const void* const* w0, const void* const*
            int64_t xbytes, int topk, const int32_t* eoff, const int32_t* elist, int nslots, int64_t N, int64_t K,
            _Float16* hout, float* fout, const float* rw, float* yacc, hipStream_t st);
 // The same products for prefill-sized batches (moe_wreg.hip): each expert's
-// weights read and decoded once per 256 slots, for the types moe_wreg_type
+// weights read and decoded once per 160 slots, for the types moe_wreg_type
 // takes on both sides, h and i multiples of 256.  xh: the tokens in fp16.
 // xf / hf: scratch of (nslots + 15 n_exp) x h (x i) fp16 values (packed
 // activations and hidden rows); with yacc null, obuf (nslots x h fp32, may
