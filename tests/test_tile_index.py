@@ -96,7 +96,7 @@ static int next(int n) { rnd = rnd * 1664525u + 1013904223u; return int((rnd >> 
 // each within [0, nslots] but of any sum, as overwritten lists can hold:
 // every accepted tile stays below moe_wreg_blocks.
 int main() {
-    // the rows fit from 16 slots per expert (where moe_wreg_shape begins), not
+    // the rows fit from 16 slots per expert (where moe_wreg_leads begins), not
     // from 14 (15 n_exp rows of padding)
     for (int e = 1; e <= 64; e++)
         for (int n = 1; n <= 1024; n++) {
@@ -139,6 +139,27 @@ int main() {
 }
 """
 
+MOE_RULE = r"""
+#include <cstdio>
+#include <initializer_list>
+#include "tile_index.hpp"
+// MoE calls that ran slower on the prefill kernels stay off them
+struct Call { bool gu, dn; int64_t t, topk, e, h; bool on; };
+int main() {
+    for (Call c : {Call{true, true, 16, 8, 8, 4096, false}, Call{true, false, 16, 8, 8, 2048, false},
+                   Call{true, true, 32, 4, 8, 4096, false}, Call{true, true, 34, 4, 8, 4096, false},
+                   Call{true, true, 36, 4, 8, 4096, true}, Call{true, false, 64, 2, 8, 4096, true},
+                   Call{false, false, 16, 8, 8, 4096, true}, Call{true, false, 500, 2, 8, 4096, true},
+                   Call{false, true, 15, 8, 8, 4096, false}, Call{true, false, 64, 1, 4, 2048, false},
+                   Call{true, false, 128, 1, 4, 2048, true}, Call{true, true, 16, 2, 8, 4096, false}})
+        if (vb::moe_wreg_leads(c.gu, c.dn, c.t, c.topk, c.e, c.h) != c.on) {
+            std::printf("%lld tokens, top-%lld of %lld\n", (long long)c.t, (long long)c.topk, (long long)c.e);
+            return 1;
+        }
+    return 0;
+}
+"""
+
 
 def _run(tmp_path, code):
     cxx = shutil.which("g++") or shutil.which("clang++")
@@ -170,3 +191,8 @@ def test_moe_tiles_stay_inside(tmp_path):
     """Expert tiles of moe_wreg.hip: any routing's tiles are all there, and
     none of overwritten lists lies past the packed blocks."""
     _run(tmp_path, MOE)
+
+
+def test_moe_rule(tmp_path):
+    """Which calls moe_wreg.hip takes: none of those that lost time on it."""
+    _run(tmp_path, MOE_RULE)

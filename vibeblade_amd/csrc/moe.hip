@@ -35,19 +35,6 @@ constexpr int MOE_MAX_EXPERTS = 64;
 constexpr int MOE_MAX_TOPK = 8;
 constexpr int MOE_MAX_SLOTS = 1024;  // tokens * topk
 
-// Whether the experts run on moe_wreg.hip, which decodes each weight once per
-// up to 160 slots but cannot fill the chip with a small down product (its
-// workgroups take 128 of the h columns of one expert).  MI355X, Q4_K gate/up
-// and Q6_K down, mean slots per expert in brackets: 8 experts of 4096 x 14336
-// 304 us against 307 at [12], 297 / 412 [16], 314 / 656 [32], 477 / 2168
-// [125]; 32 of 2048 x 4096, top-4, 190 / 201 [8], 194 / 318 [16], 212 / 510
-// [31]; 4 of 2048 x 8192 (64 down workgroups) 107 / 76 [16], 111 / 107 [25].
-bool moe_wreg_shape(int64_t slots, int64_t n_exp, int64_t h) {
-    const int64_t wgs = n_exp * (h / 128);
-    const int64_t per = wgs >= 128 ? 16 : (wgs >= 64 ? 32 : 64);
-    return slots >= per * n_exp;
-}
-
 struct ExpertPtrs {
     const uint8_t* p[MOE_MAX_EXPERTS];
 };
@@ -633,7 +620,8 @@ extern "C" int vb_moe_grouped_ffn_types(const void* const* wg, const void* const
         // expert-grouped K-split kernel (gemm_kq.hip), gate/up with the same
         // SwiGLU epilogue
         const bool wreg = moe_wreg_type(gate_up_type) && moe_wreg_type(down_type) &&
-                          moe_wreg_shape(slots, n_exp, h) && moe_wreg_fits(static_cast<int>(slots), n_exp);
+                          moe_wreg_leads(gate_up_type == TYPE_Q4_K, down_type == TYPE_Q4_K, n_tokens, topk, n_exp, h) &&
+                          moe_wreg_fits(static_cast<int>(slots), n_exp);
         if (wreg) {
             // the packed rows take obuf's place until the down product writes it
             rc = moe_wreg(gate_up_type, down_type, wg, wu, wd, n_exp, xh, static_cast<int>(slots), topk, h, i, eoff,

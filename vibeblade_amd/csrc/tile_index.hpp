@@ -1,5 +1,5 @@
-// Index arithmetic that decides which addresses a kernel touches, in plain
-// C++ (constexpr: host and device): tests/test_tile_index.py compiles this
+// Index arithmetic that decides which addresses a kernel touches, and rules of
+// dispatch on sizes alone, in plain C++ (constexpr: host and device): tests/test_tile_index.py compiles this
 // header alone for the CPU and sweeps it.
 #pragma once
 
@@ -83,6 +83,27 @@ constexpr bool moe_wreg_tile(int e, int ti, int slots, int first, int mb_max, in
     t.m0 = 16 * bb;
     t.cnt = slots - t.m0 < 16 * t.nblk ? slots - t.m0 : 16 * t.nblk;
     return t.nblk > 0 && t.blk0 + t.nblk <= cap;
+}
+
+// Where those kernels lead the 16-slot ones of moe.hip and gemm_kq.hip: they
+// decode each weight once per up to 160 slots but cannot fill the chip with a
+// small down product (its workgroups take 128 of the h columns of one expert).
+// MI355X, Q4_K gate/up and Q6_K down, us there / on the 16-slot kernels, mean
+// slots per expert in brackets, top-1 to top-8 and even to skewed routings: 8 experts of 4096 x
+// 14336 304 / 307 at [12], 297 - 402 / 367 - 454 [16], 302 - 444 / 452 - 515
+// [20], 361 - 385 / 1156 - 1177 [64]; 32 of 2048 x 4096, top-4, 190 / 201 [8],
+// 194 / 318 [16], 212 / 510 [31]; 4 of 2048 x 8192 (64 down workgroups) 107 / 76
+// [16], 98 - 154 / 111 - 214 [32].  The skinny tiles of Q4_K gate/up decode each
+// weight once as well where no expert can have more than 16 slots (top-8 of 8 at
+// [16]: 4096 x 14336, Q4_K down, 241 / 203; 2048 x 1536, Q6_K down, 52 / 48),
+// and with Q4_K down they lead up to [17] on some routings (252 / 229 at [16],
+// 267 / 258 at [17], 255 - 305 / 291 - 342 at [18]).
+constexpr bool moe_wreg_leads(bool q4k_gate_up, bool q4k_down, int64_t n_tokens, int64_t topk, int64_t n_exp, int64_t h) {
+    const int64_t wgs = n_exp * (h / 128);
+    int64_t per = wgs >= 128 ? 16 : (wgs >= 64 ? 32 : 64);
+    if (q4k_gate_up && n_tokens <= 16) return false;
+    if (q4k_gate_up && q4k_down && per < 18) per = 18;
+    return n_tokens * topk >= per * n_exp;
 }
 
 }  // namespace vb
