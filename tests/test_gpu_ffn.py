@@ -375,6 +375,25 @@ def test_moe_prefill_tiles(gu, dn, counts):
         assert O.rel_l2(yn, want) <= 5e-3, (topk, O.rel_l2(yn, want))
 
 
+@pytest.mark.parametrize("t,topk,e_n", [(9, 8, 8), (32, 8, 64), (32, 3, 5), (17, 4, 16), (64, 1, 3), (65, 1, 3),
+                                        (33, 2, 8), (33, 8, 9)])
+def test_moe_slot_lists(t, topk, e_n):
+    """The routing lists at their edges: one wave's (64 slots), one
+    workgroup's (up to 32 tokens, 256 slots) and the launch of their own."""
+    from qblocks import rand_qblocks
+    h = i = 256
+    gates, ups, downs = ([QTensor.from_bytes(rand_qblocks(Q4K, i, h, 100 * m + e), Q4K, i, h) for e in range(e_n)]
+                         for m in (1, 2, 3))
+    rng = np.random.default_rng(t + topk + e_n)
+    x = (rng.standard_normal((t, h)) * 0.01).astype(np.float32)
+    lg = rng.standard_normal((t, e_n)).astype(np.float32)
+    y, idx, w = moe_grouped_ffn(gates, ups, downs, x, lg, topk)
+    want, widx, ww = moe_oracle(gates, ups, downs, x, lg, topk)
+    assert np.array_equal(idx.cpu().numpy(), widx)
+    assert np.allclose(w.cpu().numpy(), ww, rtol=1e-5, atol=1e-6)
+    assert O.rel_l2(y.cpu().numpy(), want) <= 5e-3
+
+
 @pytest.mark.parametrize("dn", [Q4K, Q6K])
 @pytest.mark.parametrize("topk", [1, 2, 3])
 def test_moe_combine_paths(dn, topk):

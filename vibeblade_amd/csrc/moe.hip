@@ -257,14 +257,64 @@ __global__ void __launch_bounds__(256) moe_down_kernel(ExpertPtrs wd, const floa
     }
 }
 
-// ---- Q4_K experts: skinny tiles (skinny_core.hpp) --------------------------
+// ---- routing and slot lists ---------------------------------------------------
 //
 // prep: the first blocks route every token once and write the routing (ridx,
 // rw) and the slots of each expert in slot order (elist[eoff[e] ..
-// eoff[e+1]); above 64 slots moe_lists_kernel does); the others round x to fp16 (xh) -- the MFMA path rounds its
+// eoff[e+1]); with more tokens than PREP_LIST_TOKENS moe_lists_kernel writes
+// the lists); the others round x to fp16 (xh) -- the MFMA path rounds its
 // activations to fp16 anyway, and fp16 halves the activation traffic of the
 // expert kernels.
 constexpr int PREP_THREADS = 1024;
+// Up to two tokens per wave of one workgroup, which then writes the lists
+// itself: a launch less (MI355X, 1.5 to 2 us of 30 to 45 at 72 slots of 9
+// tokens); with more tokens their routing in turn would cost what it saves.
+constexpr int PREP_LIST_TOKENS = 2 * PREP_THREADS / 64;
+constexpr int PREP_LIST_SLOTS = PREP_LIST_TOKENS * MOE_MAX_TOPK;
+static_assert(MOE_MAX_SLOTS <= PREP_THREADS, "one thread per slot");
+
+// The slot lists, in slot order, by a workgroup of 1024 threads, thread q with
+// slot q's expert eq (-1: no slot): per wave a ballot per expert gives the
+// counts of its 64 slots and each slot's position among them; the counts of the
+// waves before, and of the experts before, make it the slot's place.  Slots
+// with no expert (NaN logits) are in no list.
+struct ListCounts {
+    int cnt[MOE_MAX_SLOTS / 64][MOE_MAX_EXPERTS];
+    int off[MOE_MAX_EXPERTS + 1];
+};
+__device__ __forceinline__ void slot_lists(ListCounts& l, int eq, int e_n, int32_t* __restrict__ eoff,
+                                           int32_t* __restrict__ elist) {
+    const int q = static_cast<int>(threadIdx.x), lane = q & 63, wave = q >> 6;
+    const uint64_t below = (uint64_t(1) << lane) - 1u;
+    int pos = 0, mine = 0;
+    for (int e = 0; e < e_n; e++) {
+        const uint64_t m = __ballot(eq == e);
+        if (eq == e) pos = __popcll(m & below);
+        if (lane == e) mine = __popcll(m);
+    }
+    l.cnt[wave][lane] = mine;  // lanes past the experts: 0
+    __syncthreads();
+    if (wave == 0) {  // lane e: expert e's counts to the waves' first places
+        int c = 0;
+#pragma unroll
+        for (int v = 0; v < MOE_MAX_SLOTS / 64; v++) {
+            const int x = l.cnt[v][lane];
+            l.cnt[v][lane] = c;
+            c += x;
+        }
+        int s = c;  // inclusive sum over the experts
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int a = __shfl_up(s, o, 64);
+            if (lane >= o) s += a;
+        }
+        l.off[lane] = s - c;
+        if (lane < e_n) eoff[lane] = s - c;
+        if (lane == 63) eoff[e_n] = s;
+    }
+    __syncthreads();
+    if (eq >= 0 && eq < e_n) elist[l.off[eq] + l.cnt[wave][eq] + pos] = q;
+}
 
 __global__ void __launch_bounds__(PREP_THREADS) moe_prep_kernel(
         const float* __restrict__ x, const float* __restrict__ logits, int t_n, int e_n, int topk, int64_t nx,
@@ -286,7 +336,8 @@ __global__ void __launch_bounds__(PREP_THREADS) moe_prep_kernel(
         }
         return;
     }
-    __shared__ int sexp[64];
+    __shared__ int sexp[PREP_LIST_SLOTS];
+    __shared__ ListCounts lists;
     const int nslots = t_n * topk;
     // one wave per token
     // with yzero no combine launch follows, and the routing result goes to
@@ -300,6 +351,10 @@ __global__ void __launch_bounds__(PREP_THREADS) moe_prep_kernel(
                          cw ? cw + t * topk : nullptr);
     if (rblocks > 1) return;  // the lists follow in moe_lists_kernel
     __syncthreads();
+    if (nslots > 64) {
+        slot_lists(lists, static_cast<int>(threadIdx.x) < nslots ? sexp[threadIdx.x] : -1, e_n, eoff, elist);
+        return;
+    }
     // one wave: expert e's slots are the lanes whose expert is e; a ballot
     // per expert gives its count, the running total its offset, and the
     // lanes below a slot with the same expert its position (slot order)
@@ -320,52 +375,19 @@ __global__ void __launch_bounds__(PREP_THREADS) moe_prep_kernel(
     }
 }
 
-// The slot lists of more than 64 slots (at most 1024: one thread per slot),
-// in slot order: per wave a ballot per expert gives the counts of its 64
-// slots and each slot's position among them; the counts of the waves before,
-// and of the experts before, make it the slot's place.  Slots with no expert
-// (NaN logits) are in no list.  (A loop over all slots per expert and per
-// slot, with the routing in the same single workgroup, ran 94 us at 500
-// tokens, 8 experts, top-2; the two launches 7.2 + 2.6.)
+// The lists of many tokens (at most 1024 slots), after their routing by as many
+// workgroups as it takes.  (A loop over all slots per expert and per slot, with
+// the routing in one workgroup, ran 94 us at 500 tokens, 8 experts, top-2; the
+// two launches 7.2 + 2.6.)
 __global__ void __launch_bounds__(MOE_MAX_SLOTS) moe_lists_kernel(const int32_t* __restrict__ ridx, int nslots, int e_n,
                                                                   int32_t* __restrict__ eoff,
                                                                   int32_t* __restrict__ elist) {
-    constexpr int WAVES = MOE_MAX_SLOTS / 64;
-    __shared__ int cnt[WAVES][MOE_MAX_EXPERTS];
-    __shared__ int off[MOE_MAX_EXPERTS + 1];
-    const int q = static_cast<int>(threadIdx.x), lane = q & 63, wave = q >> 6;
-    const int eq = q < nslots ? ridx[q] : -1;
-    const uint64_t below = (uint64_t(1) << lane) - 1u;
-    int pos = 0, mine = 0;
-    for (int e = 0; e < e_n; e++) {
-        const uint64_t m = __ballot(eq == e);
-        if (eq == e) pos = __popcll(m & below);
-        if (lane == e) mine = __popcll(m);
-    }
-    cnt[wave][lane] = mine;  // lanes past the experts: 0
-    __syncthreads();
-    if (wave == 0) {  // lane e: expert e's counts to the waves' first places
-        int c = 0;
-#pragma unroll
-        for (int v = 0; v < WAVES; v++) {
-            const int x = cnt[v][lane];
-            cnt[v][lane] = c;
-            c += x;
-        }
-        int s = c;  // inclusive sum over the experts
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int a = __shfl_up(s, o, 64);
-            if (lane >= o) s += a;
-        }
-        off[lane] = s - c;
-        if (lane < e_n) eoff[lane] = s - c;
-        if (lane == 63) eoff[e_n] = s;
-    }
-    __syncthreads();
-    if (eq >= 0 && eq < e_n) elist[off[eq] + cnt[wave][eq] + pos] = q;
+    __shared__ ListCounts lists;
+    slot_lists(lists, static_cast<int>(threadIdx.x) < nslots ? ridx[threadIdx.x] : -1, e_n, eoff, elist);
 }
 
+// ---- Q4_K experts: skinny tiles (skinny_core.hpp) --------------------------
+//
 // gate/up: grid (ceil(i / 64), E).  A workgroup streams 64 rows of the
 // expert's gate and up matrices once per group of 16 routed slots (the tile
 // takes super-blocks in interleaved pairs, the gate units of a pair then its
@@ -590,10 +612,11 @@ extern "C" int vb_moe_grouped_ffn_types(const void* const* wg, const void* const
     int32_t* eoff = reinterpret_cast<int32_t*>(wsb + ws.eoff);
     int32_t* elist = reinterpret_cast<int32_t*>(wsb + ws.elist);
     // 1. routing, per-expert slot lists, fp16 activations
-    // one routing workgroup and its lists up to 64 slots; above, a wave per
-    // token over as many workgroups as that takes and the lists in a launch of
-    // their own
-    const int rblocks = slots <= 64 ? 1 : static_cast<int>((n_tokens + PREP_THREADS / 64 - 1) / (PREP_THREADS / 64)) + 1;
+    // one routing workgroup and its lists up to 64 slots or PREP_LIST_TOKENS
+    // tokens; above, a wave per token over as many workgroups as that takes and
+    // the lists in a launch of their own
+    const int rblocks = slots <= 64 || n_tokens <= PREP_LIST_TOKENS
+                            ? 1 : static_cast<int>((n_tokens + PREP_THREADS / 64 - 1) / (PREP_THREADS / 64));
     const dim3 prep(static_cast<uint32_t>(rblocks + (nx / 8 + PREP_THREADS - 1) / PREP_THREADS));
     // top-k <= 2 on the quantized experts: the down kernels add each slot's
     // weighted output into y (zeroed here), so no combine launch follows
