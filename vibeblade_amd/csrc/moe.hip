@@ -266,10 +266,12 @@ __global__ void __launch_bounds__(256) moe_down_kernel(ExpertPtrs wd, const floa
 // activations to fp16 anyway, and fp16 halves the activation traffic of the
 // expert kernels.
 constexpr int PREP_THREADS = 1024;
-// Up to two tokens per wave of one workgroup, which then writes the lists
-// itself: a launch less (MI355X, 1.5 to 2 us of 30 to 45 at 72 slots of 9
-// tokens); with more tokens their routing in turn would cost what it saves.
-constexpr int PREP_LIST_TOKENS = 2 * PREP_THREADS / 64;
+// Up to 20 tokens, a little over one per wave, one workgroup routes them all and
+// writes the lists itself, a launch less.  MI355X, 32 experts of 1024 x 512, us
+// so / with moe_lists_kernel: 72 slots of 9 tokens 33.9 / 34.5, top-4 of 20
+// tokens 32.3 / 33.2, top-8 of 20 37.1 / 36.9, of 24 38.5 / 37.3, of 32 42.0 /
+// 38.1 (a round of routing is 2 to 4 us).
+constexpr int PREP_LIST_TOKENS = PREP_THREADS / 64 + 4;
 constexpr int PREP_LIST_SLOTS = PREP_LIST_TOKENS * MOE_MAX_TOPK;
 static_assert(MOE_MAX_SLOTS <= PREP_THREADS, "one thread per slot");
 
