@@ -24,7 +24,8 @@ def _more(qtype, xdt, m, n, k):
                                              (Q80, F16, 33, 4096, 4096), (Q80, F16, 224, 32768, 2048),
                                              (Q4K, F16, 224, 4096, 5120), (Q4K, F16, 17, 6144, 8192),
                                              (Q4K, F16, 33, 14336, 8192), (Q6K, F16, 256, 4096, 5120),
-                                             (Q6K, F16, 33, 4096, 6144), (Q5K, F32, 256, 14336, 3072)])
+                                             (Q6K, F16, 33, 4096, 6144), (Q5K, F32, 256, 14336, 3072),
+                                             (Q4K, F16, 17, 1536, 8192), (Q4K, F32, 17, 1536, 4864)])
 def test_wreg_leaves(qtype, xdt, m, n, k):
     assert not _more(qtype, xdt, m, n, k)
 

@@ -124,8 +124,8 @@ int64_t wreg_packed_bytes(int64_t M, int64_t K) { return (M + 15) / 16 * 16 * K 
 // N from 16 to 151936, K from 2048 to 28672, on a grid and at random; weights
 // not in cache) against the skinny, K-split or tiled kernel that the call ran
 // on before, the packing and the sum of the splits included.  No call that the
-// table takes ran below 0.97 of the other kernel's rate; they gain 2.06 in the
-// geometric mean; the ones left out are 1.14 in the mean and 0.63 at the worst.
+// table takes ran below 0.97 of the other kernel's rate; they gain 2.07 in the
+// geometric mean; the ones left out are 1.15 in the mean and 0.63 at the worst.
 // Some of both, us other / this one:
 //   fp16 X            M = 17       32           64           128          256
 //   Q4_K 4096x14336   29.5 / 21.9  35.2 / 22.3  62.8 / 25.8  77.3 / 33.8  78.7 / 49.2
@@ -139,20 +139,22 @@ int64_t wreg_packed_bytes(int64_t M, int64_t K) { return (M + 15) / 16 * 16 * K 
 //   Q4_K 14336x4096                             30.4 / 25.0  39.8 / 32.6  55.7 / 48.1
 //   Q6_K 4096x4096                              34.4 / 21.8  27.8 / 24.4  36.6 / 29.4
 // Why the lines lie there: the packing and the sum of the splits are launches
-// of their own, which a small K does not pay for; up to 64 rows with fp16 X the
+// of their own, which a small K does not pay for (called eagerly, the three
+// launches and the workspace take the host 18.5 us, one launch 11: Q4_K up to 32
+// rows begins where the other kernel takes longer than that); up to 64 rows with fp16 X the
 // other kernels decode a weight once as well; and above 192 rows the tiles of
 // 16 blocks spill 34 / 27 / 11 registers on Q5_K / Q6_K / Q8_0.
 constexpr uint8_t kWregMinSb[4][2][5][7] = {
     {
         { // Q4_K, X fp16
-            {32, 32, 32, 39,  0,  0,  0},
+            {39, 39, 39, 39,  0,  0,  0},
             {32, 24, 24, 16,  0,  8,  0},
             {32, 16, 16, 23, 16,  8,  8},
             {32, 20, 21, 27, 16,  8,  8},
             {32, 20, 39, 20, 21,  8, 10},
         },
         { // X fp32
-            {32, 16, 19, 16, 32,  0,  0},
+            {32, 24, 24, 16, 32,  0,  0},
             {32, 16, 16, 16, 13,  8,  8},
             {32, 16, 16, 16, 12,  8,  8},
             {32, 16, 16, 16, 12,  8,  8},
