@@ -345,7 +345,7 @@ def test_moe_more_types(gu, dn):
 @pytest.mark.parametrize("counts", [(300, 1, 0, 83), (256, 129, 112, 15), (33, 48, 65, 192), (64, 160, 100, 20)])
 def test_moe_prefill_tiles(gu, dn, counts):
     """Prefill-sized batches: every tile height of the expert-grouped kernels
-    (1 .. 16 blocks of 16 slots, experts split into two tiles, an idle expert,
+    (1 .. 10 blocks of 16 slots, experts split into two tiles, an idle expert,
     last blocks with 1 to 16 live rows), a gate/up K of one and a down K of
     three super-blocks; with top-2 and top-3 a random routing.  The bound is
     the other MoE tests': fp16 operands and hidden rows."""

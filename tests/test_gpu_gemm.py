@@ -190,8 +190,9 @@ def test_tiled_tile_configs(knob, cfg):
 @pytest.mark.parametrize("m", [17, 64, 100, 128, 129, 256])
 def test_mid_m_at_config_shape(m):
     """The mid-M sizes of speculative verify and chunked prefill at
-    N = 14336, K = 4096 (fp16 X with 0.1 % outliers x20), on the default tile
-    for each M."""
+    N = 14336, K = 4096 (fp16 X with 0.1 % outliers x20): gemm()'s kernel for
+    each M, and the one that vb_gemm runs without a workspace (from M = 100 on
+    the tiled kernel with its default tile)."""
     n, k = 14336, 4096
     gen = torch.Generator(device="cuda").manual_seed(m)
     qt = QTensor.quantize(torch.randn((n, k), generator=gen, device="cuda") * 0.02, Q4K)
@@ -201,6 +202,10 @@ def test_mid_m_at_config_shape(m):
     y = gemm(qt, xh).cpu().numpy()
     want = ref_gemm(qt, xh.float().cpu().numpy())
     assert O.rel_l2(y, want) <= TOL
+    out = torch.empty((m, n), dtype=torch.float32, device="cuda")
+    assert _lib.load().vb_gemm(qt.ptr(), xh.data_ptr(), 1, out.data_ptr(), m, n, k, Q4K, 0,
+                               torch.cuda.current_stream().cuda_stream) == 0
+    assert O.rel_l2(out.cpu().numpy(), want) <= TOL
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 16, 256), (257, 113, 512), (300, 257, 1024), (512, 224, 4096),
@@ -844,8 +849,8 @@ def test_q5k_xreg(m, n, k):
                                    (129, 300, 1280), (145, 33, 512), (161, 300, 2304), (193, 96, 256),
                                    (256, 300, 3328)])
 def test_wreg(knob, qtype, m, n, k):
-    """The register-decoding kernel (gemm_wreg.hip) at every tile height, row
-    tiles, K splits of unequal length (13, 9 and 10 super-blocks), K groups
+    """The register-decoding kernel (gemm_wreg.hip) in tiles of 1 to 4 blocks,
+    row tiles, K splits of unequal length (13, 9 and 10 super-blocks), K groups
     with nothing to do (one super-block) and ragged N, both X types."""
     knob("VB_GEMM_WREG_MIN_M", "2")
     lib = _lib.load()
@@ -861,21 +866,52 @@ def test_wreg(knob, qtype, m, n, k):
         assert O.rel_l2(y, ref_gemm(qt, xt.float().cpu().numpy())) <= TOL, dtype
 
 
+@pytest.mark.parametrize("qtype", [Q4K, ggml.GGML_TYPE_Q5_K, Q6K, Q80])
+@pytest.mark.parametrize("n,k,ks", [(16400, 512, 1), (8200, 2304, 2)])
+def test_wreg_tall(knob, qtype, n, k, ks):
+    """Tiles of 5 to 16 blocks (all the rows in one, as the columns and K splits
+    take more than half of the CUs), ragged in rows and columns, with and
+    without K splits, both X types."""
+    knob("VB_GEMM_WREG_MIN_M", "2")
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert 2 * (n + 127) // 128 * ks > cus  # no room for a second row tile
+    ms = [65, 96, 97, 128, 144, 160, 161, 180, 200, 256]  # 5 to 13 and 16 blocks
+    if qtype == ggml.GGML_TYPE_Q5_K:
+        qt, x = make_other(qtype, n, k, n), make(max(ms), 1, k, n)[1]
+    else:
+        qt, x = make(max(ms), n, k, n + qtype, qtype=qtype)
+    for dtype in (torch.float16, torch.float32):
+        xt = torch.from_numpy(x).to("cuda", dtype)
+        want = ref_gemm(qt, xt.float().cpu().numpy())
+        for m in ms:
+            y = gemm(qt, xt[:m]).cpu().numpy()
+            assert np.all(np.isfinite(y))
+            assert O.rel_l2(y, want[:m]) <= TOL, (dtype, m)
+
+
 @pytest.mark.parametrize("qtype,m,n,k,dtype", [(Q4K, 100, 1024, 14336, torch.float16),
                                                (Q6K, 33, 300, 8192, torch.float16),
                                                (Q80, 8, 300, 12288, torch.float32),
                                                (Q6K, 300, 14336, 512, torch.float32),
-                                               (Q4K, 600, 1000, 4096, torch.float32)])
+                                               (Q4K, 600, 1000, 4096, torch.float32)]
+                         + [(t, 300, 520, 8192, torch.float32) for t in [ggml.GGML_TYPE_Q5_K, Q80] + B32_TYPES]
+                         + [(t, 1000, 7000, 2560, torch.float16) for t in [ggml.GGML_TYPE_Q5_K] + B32_TYPES])
 def test_scratch_routes(qtype, m, n, k, dtype):
-    """Routes that vb_gemm_scratch opens: the register-decoding kernel and
-    fp32 X on the packed-X kernel.  Without a workspace, and with one that is
-    a byte short, the call still runs, and all agree."""
+    """Routes that vb_gemm_scratch opens: the register-decoding kernel, fp32 X
+    on the packed-X kernel for every type of it (with K splits at N = 520 and
+    1000) and fp16 X below N = 8192 for the slowly decoded ones.  Without a
+    workspace, and with one that is a byte short, the call still runs, and all
+    agree."""
     lib = _lib.load()
-    qt, x = make(m, n, k, m + n, qtype=qtype)
+    if qtype in (Q4K, Q6K, Q80):
+        qt, x = make(m, n, k, m + n, qtype=qtype)
+    else:
+        qt, x = make_other(qtype, n, k, m + n), make(m, 1, k, m)[1]
     xt = torch.from_numpy(x).to("cuda", dtype)
     xdt = 1 if dtype == torch.float16 else 0
     need = lib.vb_gemm_scratch(m, n, k, qtype, xdt, 0)
-    assert need > lib.vb_gemm_workspace(m, n, k, qtype, xdt, 0)
+    # (Q5_0 / Q5_1 ask for their weights in fp16 in any case: that may be enough)
+    assert need > lib.vb_gemm_workspace(m, n, k, qtype, xdt, 0) or qtype in B32_TYPES[2:]
     want = ref_gemm(qt, xt.float().cpu().numpy())
     y = gemm(qt, xt).cpu().numpy()
     assert O.rel_l2(y, want) <= TOL
@@ -953,3 +989,21 @@ def test_no_room_for_scratch(monkeypatch, qtype, m, n, k, dtype):
     assert refused == [nb]
     # the same fp16 operands in another order of fp32 sums
     assert O.rel_l2(y.cpu().numpy(), want) <= 1e-5
+
+
+@pytest.mark.parametrize("qtype,n,k", [(ggml.GGML_TYPE_Q5_K, 12301, 4096), (Q6K, 12301, 4096), (Q80, 12301, 4096),
+                                       (ggml.GGML_TYPE_Q5_K, 2050, 2048), (Q6K, 24601, 1024), (Q80, 24601, 1280)])
+def test_rows_default(qtype, n, k):
+    """The row-streaming kernel where variant 0 takes it: full images (K =
+    4096), one to seven groups of rows per workgroup, a ragged last one."""
+    if qtype == ggml.GGML_TYPE_Q5_K:
+        qt, x = make_other(qtype, n, k, n), make(16, 1, k, n)[1]
+    else:
+        qt, x = make(16, n, k, n + qtype, qtype=qtype)
+    for dtype in (torch.float16, torch.float32):
+        xt = torch.from_numpy(x).to("cuda", dtype)
+        want = ref_gemm(qt, xt.float().cpu().numpy())
+        for m in (5, 16):
+            y = gemm(qt, xt[:m]).cpu().numpy()
+            assert np.all(np.isfinite(y))
+            assert O.rel_l2(y, want[:m]) <= TOL, (dtype, m)
