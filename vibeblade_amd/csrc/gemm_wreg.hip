@@ -117,15 +117,15 @@ int64_t wreg_packed_bytes(int64_t M, int64_t K) { return (M + 15) / 16 * 16 * K 
 }  // namespace
 
 // Where this kernel leads: the smallest K, in super-blocks, from which it does
-// at every K measured (0: not taken), by the rows of X (up to 32, 64, 128, 192,
-// 256) and the columns (N up to 511, 2047, 4096, 8191, 16384, 32768, more).
+// at every K measured (0: not taken), by the rows of X (kWregRows) and the
+// columns (kWregCols; the last entry beyond).
 //
 // Measured on MI355X over 68000 calls (each type and X; 11 to 19 values of M;
 // N from 16 to 151936, K from 2048 to 28672, on a grid and at random; weights
 // not in cache) against the skinny, K-split or tiled kernel that the call ran
 // on before, the packing and the sum of the splits included.  No call that the
-// table takes ran below 0.97 of the other kernel's rate; they gain 2.07 in the
-// geometric mean; the ones left out are 1.15 in the mean and 0.63 at the worst.
+// table takes ran below 0.97 of the other kernel's rate; they gain 2.05 in the
+// geometric mean; the ones left out are 1.09 in the mean and 0.63 at the worst.
 // Some of both, us other / this one:
 //   fp16 X            M = 17       32           64           128          256
 //   Q4_K 4096x14336   29.5 / 21.9  35.2 / 22.3  62.8 / 25.8  77.3 / 33.8  78.7 / 49.2
@@ -140,73 +140,91 @@ int64_t wreg_packed_bytes(int64_t M, int64_t K) { return (M + 15) / 16 * 16 * K 
 //   Q6_K 4096x4096                              34.4 / 21.8  27.8 / 24.4  36.6 / 29.4
 // Why the lines lie there: the packing and the sum of the splits are launches
 // of their own, which a small K does not pay for (called eagerly, the three
-// launches and the workspace take the host 18.5 us, one launch 11: Q4_K up to 32
-// rows begins where the other kernel takes longer than that); up to 64 rows with fp16 X the
-// other kernels decode a weight once as well; and above 192 rows the tiles of
-// 16 blocks spill 34 / 27 / 11 registers on Q5_K / Q6_K / Q8_0.
-constexpr uint8_t kWregMinSb[4][2][5][7] = {
+// launches and the workspace take the host 18.5 us, one launch 11: Q4_K up to 20
+// rows begins where the other kernel takes longer than that); up to 64 rows with
+// fp16 X the other kernels decode a weight once as well; and above 192 rows the
+// tiles of 16 blocks spill 34 / 27 / 11 registers on Q5_K / Q6_K / Q8_0.
+constexpr int kWregRows[7] = {20, 32, 40, 64, 128, 192, 256};
+constexpr int kWregCols[8] = {511, 2047, 4096, 6144, 8191, 11264, 16384, 32768};
+constexpr uint8_t kWregMinSb[4][2][7][9] = {
     {
         { // Q4_K, X fp16
-            {39, 39, 39, 39,  0,  0,  0},
-            {32, 24, 24, 16,  0,  8,  0},
-            {32, 16, 16, 23, 16,  8,  8},
-            {32, 20, 21, 27, 16,  8,  8},
-            {32, 20, 39, 20, 21,  8, 10},
+            {39, 39, 39, 39, 39,  0,  0,  0,  0},
+            {32, 32, 32, 32, 34,  0,  0,  0,  0},
+            {32, 24, 24, 16, 16, 47,  0,  8,  0},
+            {32, 16, 16, 16, 16, 32, 32,  8,  8},
+            {32, 16, 16, 17, 23, 16, 16,  8,  8},
+            {32, 20, 21, 29, 22, 16, 16,  8,  8},
+            {32, 20, 39, 20, 22, 16, 21,  8, 10},
         },
         { // X fp32
-            {32, 24, 24, 16, 32,  0,  0},
-            {32, 16, 16, 16, 13,  8,  8},
-            {32, 16, 16, 16, 12,  8,  8},
-            {32, 16, 16, 16, 12,  8,  8},
-            {32, 16, 16, 16, 14,  8,  8},
+            {32, 24, 24, 16, 16, 32, 32,  0,  0},
+            {32, 16, 16, 16, 16, 32, 32,  0, 32},
+            {32, 16, 16, 16, 16, 12, 12,  8,  8},
+            {32, 16, 16, 16, 16, 15, 13,  8,  8},
+            {32, 16, 16, 16, 16, 12, 12,  8,  8},
+            {32, 16, 16, 16, 16, 12, 12,  8,  8},
+            {32, 16, 16, 16, 16, 15, 14,  8,  8},
         },
     },
     {
         { // Q5_K, X fp16
-            {48, 50, 52, 32, 21, 12,  0},
-            {32, 31, 32, 16, 12,  8,  8},
-            {32, 16, 16, 16, 14,  8,  8},
-            {32, 20, 20, 20, 13, 10,  8},
-            {32, 20, 30, 39,  0,  0,  0},
+            {48, 50, 52, 32, 34, 15, 21, 12,  0},
+            {32, 35, 41, 32, 34, 12, 20, 12, 12},
+            {32, 31, 32, 16, 16, 12, 12,  8,  8},
+            {32, 20, 20, 16, 16, 12, 12,  8,  8},
+            {32, 16, 16, 16, 16, 15, 14,  8,  8},
+            {32, 20, 20, 20, 22, 12, 13, 10,  8},
+            {32, 20, 30, 20, 39, 29,  0,  0,  0},
         },
         { // X fp32
-            {32, 32, 32, 32, 13, 12, 12},
-            {32, 16, 16, 16, 12,  8,  8},
-            {32, 16, 16, 16, 12,  8,  8},
-            {32, 16, 16, 16, 12,  8,  8},
-            {32, 16, 27, 16, 23,  0,  0},
+            {32, 32, 32, 32, 34, 12, 13, 12, 12},
+            {32, 32, 32, 32, 34, 12, 12, 12, 12},
+            {32, 16, 16, 16, 16, 12, 12,  8,  8},
+            {32, 16, 16, 16, 16, 12, 12,  8,  8},
+            {32, 16, 16, 16, 16, 12, 12,  8,  8},
+            {32, 16, 16, 16, 16, 12, 12,  8,  8},
+            {32, 16, 27, 16, 16, 12, 23, 42,  0},
         },
     },
     {
         { // Q6_K, X fp16
-            {48, 50, 52, 48, 48,  0,  0},
-            {32, 31, 32, 24, 24,  8,  0},
-            {32, 16, 16, 20, 16,  8,  8},
-            {32, 20, 20, 20, 20, 20, 20},
-            {32, 20, 32, 20, 25,  0,  0},
+            {48, 50, 52, 48, 50, 48, 48,  0,  0},
+            {48, 48, 48, 48, 50, 48, 48,  0,  0},
+            {32, 31, 32, 24, 25, 24, 24,  8,  0},
+            {32, 24, 24, 24, 25, 24, 24,  8,  9},
+            {32, 16, 16, 20, 22, 16, 16,  8,  8},
+            {32, 20, 20, 22, 22, 20, 20, 20, 20},
+            {32, 20, 32, 20, 22, 25, 20,  0,  0},
         },
         { // X fp32
-            {32, 32, 32, 32, 32,  0,  0},
-            {32, 16, 16, 16, 12,  8,  8},
-            {32, 16, 16, 16, 12,  8,  8},
-            {32, 16, 16, 16, 12,  8,  8},
-            {32, 16, 16, 16, 14,  0,  0},
+            {32, 32, 32, 32, 34, 32, 32,  0,  0},
+            {32, 32, 32, 32, 34, 32, 32,  0, 32},
+            {32, 16, 16, 16, 16, 12, 12,  8,  8},
+            {32, 16, 16, 16, 16, 12, 12,  8,  8},
+            {32, 16, 16, 16, 16, 12, 12,  8,  8},
+            {32, 16, 16, 16, 16, 12, 12,  8,  8},
+            {32, 16, 16, 16, 16, 12, 14, 42,  0},
         },
     },
     {
         { // Q8_0, X fp16
-            {48, 50, 47, 32, 14, 12, 16},
-            {32, 31, 30, 16, 13,  8, 10},
-            {32, 16, 16, 19, 14,  8,  8},
-            {32, 20, 20, 23, 14, 10, 10},
-            {32, 20, 30, 27, 25,  0,  0},
+            {48, 50, 47, 32, 34, 15, 14, 12, 16},
+            {32, 35, 35, 32, 34, 12, 13, 12, 12},
+            {32, 31, 30, 16, 16, 12, 13,  8, 10},
+            {32, 20, 20, 16, 16, 12, 12,  8,  8},
+            {32, 16, 16, 16, 22, 15, 14,  8,  8},
+            {32, 20, 20, 24, 22, 15, 14, 10, 10},
+            {32, 20, 30, 20, 27, 25, 21,  0,  0},
         },
         { // X fp32
-            {32, 32, 32, 32, 12, 12, 12},
-            {32, 16, 16, 16, 12,  8,  8},
-            {32, 16, 16, 16, 12,  8,  8},
-            {32, 16, 16, 20, 12,  8,  8},
-            {32, 16, 16, 16, 14,  0,  0},
+            {32, 32, 32, 32, 34, 12, 12, 12, 12},
+            {32, 32, 32, 32, 34, 12, 12, 12, 12},
+            {32, 16, 16, 16, 16, 12, 12,  8,  8},
+            {32, 16, 16, 16, 16, 12, 12,  8,  8},
+            {32, 16, 16, 16, 16, 12, 12,  8,  8},
+            {32, 16, 16, 20, 16, 12, 12,  8,  8},
+            {32, 16, 16, 16, 16, 12, 14, 22, 20},
         },
     },
 };
@@ -219,8 +237,9 @@ bool gemm_wreg_shape(int32_t type, int32_t x_dtype, int64_t M, int64_t N, int64_
     // few rows: the conversion of fp32 X alone makes it worth it (M = 8, 4096 x
     // 12288: Q4_K 25.9 / 20.5, Q8_0 32.0 / 28.2)
     if (M < 17) return f32 && M >= 8 && N < 8192 && K >= (type == TYPE_Q6_K ? 14336 : 12288);
-    const int m = M <= 32 ? 0 : (M <= 64 ? 1 : (M <= 128 ? 2 : (M <= 192 ? 3 : 4)));
-    const int n = N <= 511 ? 0 : (N <= 2047 ? 1 : (N <= 4096 ? 2 : (N <= 8191 ? 3 : (N <= 16384 ? 4 : (N <= 32768 ? 5 : 6)))));
+    int m = 0, n = 0;
+    while (M > kWregRows[m]) m++;
+    while (n < 8 && N > kWregCols[n]) n++;
     const int64_t sb = kWregMinSb[t][f32 ? 1 : 0][m][n];
     return sb != 0 && K >= 256 * sb;
 }
