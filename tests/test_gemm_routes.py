@@ -39,7 +39,7 @@ def test_wreg_takes(qtype, xdt, m, n, k):
 
 
 @pytest.mark.parametrize("qtype,xdt,m,n,k", [(Q80, F32, 257, 3000, 1536), (Q5K, F32, 300, 2048, 2048),
-                                             (Q6K, F32, 300, 8200, 512), (Q4K, F32, 257, 4096, 1024),
+                                             (Q6K, F32, 300, 2048, 2048), (Q4K, F32, 257, 4096, 1024),
                                              (Q4K, F32, 513, 9871, 4096), (Q4K, F32, 1024, 8192, 1024),
                                              (Q5K, F16, 2048, 4096, 5120), (Q40, F16, 1024, 8191, 4096),
                                              (Q40, F32, 300, 3000, 1536)])

@@ -745,38 +745,55 @@ int gemm_other(const void* w, const void* X, int32_t x_dtype, float* Y, int64_t 
     return rc;
 }
 
+// Estimates, in us, for the rule below.  Both kernels take whole rounds of tiles
+// over the CUs, each a time per element of K.  Tiled: by tile, as measured (the
+// median of t / K is within 10 % of it for six types at one to eight rounds);
+// Q5_0 / Q5_1 decode their weights to fp16 first.  Packed-X: its rounds (17 ns
+// an element) over the K splits, the sum of these, and the packing of X.
+static double tiled_est(int32_t type, int32_t x_dtype, int64_t M, int64_t N, int64_t K) {
+    const TileCfg c = tiled_cfg(type, x_dtype, M, N, K);
+    const double ns = c.wm == 4 ? 20.0 : (c.wm == 1 ? 7.6 : (c.wn == 4 ? 16.5 : (c.ks == 2 ? 9.0 : 11.6)));
+    const int64_t rounds = (tile_count(c, M, N) + num_cus() - 1) / num_cus();
+    return 3 + 1e-3 * K * ns * (rounds > 1 ? 0.93 : 1.0) * rounds + (gemm_b32_high(type) ? 4 + N * K / 1.3e6 : 0);
+}
+static double xr_est(int32_t x_dtype, int64_t M, int64_t N, int64_t K, int ks) {
+    const double pack = 4 + M * K * (x_dtype == X_F32 ? 6 : 4) / 3e6;
+    return pack + 17e-3 * K * gemm_xr_rounds(M, N, ks) / ks + (ks > 1 ? 3 + ks * M * N * 8 / 4e6 : 0);
+}
+
 // The packed-X kernel beyond the shapes whose workspace vb_gemm_workspace
 // states, with the splits of gemm_xr_ksplit_even: fp32 X (the tiled kernel
 // converts it once per column tile), and fp16 X at N < 8192 for the types
 // whose other kernels decode slowly (Q4_K, Q6_K and Q8_0 keep the tiled kernel
-// there: Q8_0 7943 x 8448 at M = 845 169 us tiled / 201).  A short K does not
-// pay for the packing unless the rounds of workgroups fill the CUs (`busy`, in
-// percent); a long one mostly does in any case.  MI355X, 40000 calls timed (M
-// from 257 to 4096, K from 256 to 28672), rate against the kernel that the
-// call ran on before, the least and the geometric mean:
-//   fp32 X, the types but Q4_K   taken 0.92, 1.68 - 1.96   left out 0.55, 1.1 - 1.3
-//   fp32 X, Q4_K                 taken 0.93, 1.75          left out 0.68, 1.2
-//   fp16 X, Q4_0 / Q4_1          taken 0.89, 1.6           left out 0.70, 1.4
-//   fp16 X, Q5_K / Q5_0 / Q5_1   taken 0.93, 1.42 - 1.48   left out 0.65, 1.2 - 1.3
+// there: Q8_0 7943 x 8448 at M = 845 169 us tiled / 201).  It is taken where the
+// tiled kernel's estimate is `margin` percent of its own or more; the margin
+// makes up for what a type's decode costs either kernel.  MI355X, 50000 calls
+// timed (M from 257 to 4096, K from 256 to 28672), rate against the kernel that
+// the call ran on before, least and geometric mean of those taken, and how many
+// of those left out would have gained more than 3 %:
+//   fp32 X  Q4_K 0.88, 1.68, 151 of 388     Q5_K / Q6_K / Q8_0 0.90, 1.70, 659 of 1305
+//           Q4_0 / Q4_1 0.94, 1.91, 370 of 598         Q5_0 / Q5_1 0.93, 1.80, 139 of 196
+//   fp16 X  Q4_0 / Q4_1 0.93, 1.63, 184 of 400   Q5_K 0.86, 1.47, 25 of 92   Q5_0 / Q5_1
+//           0.91, 1.33, 52 of 269
 // Some of them, us before / packed-X: fp32 X, Q6_K 4096 x 14336 at M = 777
-// 250 / 159, 3000 x 1536 at 300 17.6 / 28.0 (left out: 30 % busy), Q4_K 14336 x
-// 4096 at 512 94 / 64, 9871 x 4096 at 513 83 / 110 (left out: 52 % busy), Q8_0
-// 2048 x 2048 at 300 19.0 / 25.6 (left out: 30 %); fp16 X, Q4_0 5461 x 12288 at
-// 533 229 / 131, Q5_K 4096 x 5120 at 2048 95 / 130 (left out: 5 splits).
+// 250 / 159, Q4_K 14336 x 4096 at 512 94 / 64; left out: Q6_K 3000 x 1536 at 300
+// 17.6 / 28.0, Q4_K 9871 x 4096 at 513 83 / 110, Q8_0 2048 x 2048 at 300 19.0 /
+// 25.6; fp16 X, Q4_0 5461 x 12288 at 533 229 / 131; left out: Q5_K 4096 x 5120 at
+// 2048 95 / 130.
 static bool xr_even_shape(int32_t type, int32_t x_dtype, int64_t M, int64_t N, int64_t K) {
     if (!gemm_xr_type(type) || M <= 256 || M > INT32_MAX || K % 256 != 0) return false;
-    const bool b32 = gemm_b32_type(type), q4k = type == TYPE_Q4_K;
-    if (!b32 && !q4k && type != TYPE_Q5_K && !knobs().gemm_xr_kq) return false;
-    const int ks = gemm_xr_ksplit_even(M, N, K), busy = gemm_xr_busy(M, N, ks);
-    if (x_dtype == X_F32) {
-        if (N * K < 4000000) return false;
-        if (q4k && N < 8192) return M <= 768 && (K >= 4096 || busy >= 90);
-        if (q4k) return busy >= 90 || (N > 16384 && K >= 2048);
-        return K >= 4096 || (N >= 8192 && K >= 2048) || busy >= (K >= 1024 ? 70 : 80);
+    const bool b32 = gemm_b32_type(type), high = gemm_b32_high(type), f32 = x_dtype == X_F32;
+    if (!b32 && type != TYPE_Q4_K && type != TYPE_Q5_K && !knobs().gemm_xr_kq) return false;
+    if (f32) {
+        if (N * K < 4000000 || (type == TYPE_Q4_K && N < 8192 && M > 768)) return false;
+    } else {
+        if (N >= 8192 || gemm_xr_ksplit(M, N, K) > 1) return false;
+        if (!(b32 && N * K >= 8000000) && !(type == TYPE_Q5_K && N * K >= 16000000)) return false;
     }
-    if (N >= 8192 || gemm_xr_ksplit(M, N, K) > 1) return false;
-    if (b32 && !gemm_b32_high(type)) return N * K >= 8000000 && busy >= (M <= 1024 ? 80 : 90);
-    return (b32 || type == TYPE_Q5_K) && N * K >= (b32 ? 8000000 : 16000000) && busy >= 80 && ks <= 2;
+    const int margin = type == TYPE_Q4_K ? 80
+                     : high ? (f32 ? 100 : (type == TYPE_Q5_1 ? 115 : 105))
+                     : b32 ? (f32 ? 90 : 95) : (f32 ? 95 : 100);
+    return 100 * tiled_est(type, x_dtype, M, N, K) >= margin * xr_est(x_dtype, M, N, K, gemm_xr_ksplit_even(M, N, K));
 }
 
 int gemm_dispatch(const void* w, const void* X, int32_t x_dtype, float* Y, int64_t M, int64_t N, int64_t K,

@@ -563,10 +563,10 @@ int gemm_xr_ksplit_even(int64_t M, int64_t N, int64_t K) {
     return best;
 }
 
-// Percent of the CUs that the workgroups keep busy over their whole rounds.
-int gemm_xr_busy(int64_t M, int64_t N, int ks) {
-    const int64_t wgs = (N + 16 * XR_NF - 1) / (16 * XR_NF) * ((M + XR_TM - 1) / XR_TM) * ks, cus = num_cus();
-    return static_cast<int>(100 * wgs / ((wgs + cus - 1) / cus * cus));
+// Whole rounds of workgroups over the CUs.
+int64_t gemm_xr_rounds(int64_t M, int64_t N, int ks) {
+    const int64_t wgs = (N + 16 * XR_NF - 1) / (16 * XR_NF) * ((M + XR_TM - 1) / XR_TM) * ks;
+    return (wgs + num_cus() - 1) / num_cus();
 }
 
 int gemm_ksum(const float* P, float* Y, int64_t total, int ks, hipStream_t st) {

@@ -157,7 +157,7 @@ int gemm_ksum(const float* P, float* Y, int64_t total, int ks, hipStream_t st);
 int tiled_zsplit(int type, int x_dtype, int64_t M, int64_t N, int64_t K);
 int64_t gemm_xr_workspace(int64_t M, int64_t N, int64_t K);
 int gemm_xr_ksplit_even(int64_t M, int64_t N, int64_t K);
-int gemm_xr_busy(int64_t M, int64_t N, int ks);
+int64_t gemm_xr_rounds(int64_t M, int64_t N, int ks);
 int64_t gemm_xr_workspace(int64_t M, int64_t N, int64_t K, int ks);
 // n_rows x k of W (a decodable type other than F16) as row-major fp16 at out,
 // each value rounded once (dequant.hip; k % 4 == 0, out 16-byte aligned).
