@@ -194,8 +194,8 @@ int64_t vb_gemm_workspace(int64_t m, int64_t n, int64_t k, int32_t ggml_type, in
 /* The workspace with which vb_gemm_ws runs variant `variant` at its best: at
  * least vb_gemm_workspace, and more where a kernel that could do without one
  * is beaten by one that packs X or splits K (variant 0: Q4_K / Q5_K / Q6_K /
- * Q8_0 up to m = 256 where gemm_wreg.hip leads, fp32 X on the packed-X kernel
- * above).  vb_gemm_ws
+ * Q8_0 up to m = 256 where gemm_wreg.hip leads; above, fp32 X, and fp16 X of
+ * the slowly decoded types, where the packed-X kernel leads).  vb_gemm_ws
  * accepts any size: with less it runs the kernels that fit. */
 int64_t vb_gemm_scratch(int64_t m, int64_t n, int64_t k, int32_t ggml_type, int32_t x_dtype, int32_t variant);
 int vb_gemm_ws(const void* w, const void* x, int32_t x_dtype, float* y, int64_t m, int64_t n, int64_t k,

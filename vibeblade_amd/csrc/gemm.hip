@@ -776,7 +776,7 @@ static double xr_est(int32_t x_dtype, int64_t M, int64_t N, int64_t K, int ks) {
 //   fp16 X  Q4_0 / Q4_1 0.93, 1.63, 184 of 400   Q5_K 0.86, 1.47, 25 of 92   Q5_0 / Q5_1
 //           0.91, 1.33, 52 of 269
 // Some of them, us before / packed-X: fp32 X, Q6_K 4096 x 14336 at M = 777
-// 250 / 159, Q4_K 14336 x 4096 at 512 94 / 64; left out: Q6_K 3000 x 1536 at 300
+// 252 / 171, Q4_K 14336 x 4096 at 512 94 / 64; left out: Q6_K 3000 x 1536 at 300
 // 17.6 / 28.0, Q4_K 9871 x 4096 at 513 83 / 110, Q8_0 2048 x 2048 at 300 19.0 /
 // 25.6; fp16 X, Q4_0 5461 x 12288 at 533 229 / 131; left out: Q5_K 4096 x 5120 at
 // 2048 95 / 130.

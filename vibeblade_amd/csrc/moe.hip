@@ -12,7 +12,10 @@
 // Four launches, no host round trip:
 //   1. prep: routes every token once (routing written for the combine and the
 //      caller), lists the slots (token * topk + k) of each expert in slot
-//      order, and rounds x to fp16.
+//      order, and rounds x to fp16 (above 64 slots and 20 tokens the lists are
+//      a launch of their own).
+//   Prefill-sized batches of Q4_K / Q5_K / Q6_K / Q8_0 experts (moe_wreg_leads)
+//   then run moe_wreg.hip; the others:
 //   2. gate/up.  Q4_K experts: grid (i/64, E), skinny tiles (skinny_core.hpp)
 //      of 64 gate and 64 up rows per 16 slots, silu(g) * u written as fp16
 //      into hbuf.  F32 experts: grid (i/16, E), 16-row tiles on
@@ -21,7 +24,7 @@
 //      output of every slot into obuf.
 //   4. combine: y_t = sum_k w_tk * obuf[t*topk + k] in slot order (fixed
 //      order, deterministic); also copies the routing to (indices, weights).
-// Each expert's weights are streamed once per 16 routed slots.
+// These stream each expert's weights once per 16 routed slots.
 #include "mfma_q4k.hpp"
 #include "skinny_core.hpp"
 #include "tile_index.hpp"
@@ -380,7 +383,7 @@ __global__ void __launch_bounds__(PREP_THREADS) moe_prep_kernel(
 // The lists of many tokens (at most 1024 slots), after their routing by as many
 // workgroups as it takes.  (A loop over all slots per expert and per slot, with
 // the routing in one workgroup, ran 94 us at 500 tokens, 8 experts, top-2; the
-// two launches 7.2 + 2.6.)
+// two launches 7.2 + 4.7.)
 __global__ void __launch_bounds__(MOE_MAX_SLOTS) moe_lists_kernel(const int32_t* __restrict__ ridx, int nslots, int e_n,
                                                                   int32_t* __restrict__ eoff,
                                                                   int32_t* __restrict__ elist) {

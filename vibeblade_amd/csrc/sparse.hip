@@ -1477,7 +1477,9 @@ extern "C" int vb_ema_predict(const float* probs, const float* gate_values, int6
     const int flags = (warm ? PRED_WARM : 0) | (gate_values ? PRED_GATE : 0) | (combined ? PRED_COMBINED : 0);
     const int ni = static_cast<int>(n);
     hipStream_t st = as_stream(stream);
-    // warm and no gate in it: values in registers up to n = 32768; else values
+    // warm and no gate in it: values in registers up to n = 32768 (32 of them a
+    // thread spill 24 registers; still 2.4 to 9.5 times as fast as the streaming
+    // kernel: n = 18944, k = 1894 94 / 29 us, 32768, 3276 130 / 33); else values
     // in LDS for n <= 16384, the streaming kernel above
     if (warm && !combined && n <= 1024 * 32) {
         auto go = [&](auto per_c) {

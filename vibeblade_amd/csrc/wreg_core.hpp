@@ -1,6 +1,7 @@
 // GEMM tile with the weights decoded straight into B fragments in registers
 // and the activations shared through LDS, for 17 to 256 activation rows per
-// tile; used by the expert-grouped MoE products (moe_wreg.hip).
+// tile; used by the batched GEMM (gemm_wreg.hip) and the expert-grouped MoE
+// products (moe_wreg.hip, up to 160 rows).
 //
 // Why this shape.  At these row counts a weight serves few enough MFMAs that
 // decoding it costs about as much as multiplying it, so each weight is
@@ -12,13 +13,15 @@
 // workgroup has four such waves per K group; two workgroups (or two K
 // groups) fill a CU, so one wave's decode runs beside another's MFMAs.
 //
-// What bounds it (MI355X, 8 experts of 4096 x 14336, Q4_K gate/up and Q6_K
-// down, 125 slots each: gate/up 260 us, 900 TFLOP/s; down 220 us): the MFMAs
-// with their barriers alone 150 / 103 us, their LDS reads 42 / 15 more, the
-// decode 55 / 83 and the waits for weights 50 / 43 (timing copies without
-// each); spelling out the order of reads, MFMAs and decode took 300 / 240 to
-// 260 / 220.  At 25 to 64 slots per expert the weight loads bound it, at
-// about 3 TB/s: a load touches 16 rows.
+// What bounds it (MI355X, kernel trace and counters, the GEMM case 100 rows of
+// 4096 x 14336 Q4_K, the MoE 8 experts of 4096 x 14336, Q4_K gate/up and Q6_K
+// down, 125 slots each): GEMM 23.5 us, gate/up 282 (830 TFLOP/s), down 243.
+// The matrix cores are busy 18 / 45 / 23 % of that, a wave waits 40 / 20 / 35 %
+// of its life and issues 26 / 33 / 19 %: MFMA, decode and the waits for weights
+// come in turn more than beside each other.  No LDS bank conflicts.  Spelling
+// out the order of reads, MFMAs and decode took gate/up / down from 300 / 240 to
+// 260 / 220.  At 25 to 64 slots per expert the weight loads bound it, at about
+// 3 TB/s: a load touches 16 rows.
 //
 // K order.  Lane group g (lane / 16) of the MFMA takes its own 64 of a
 // super-block's 256 elements, so a lane loads whole 16-byte pieces of its
